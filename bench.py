@@ -189,9 +189,9 @@ def forward_bench(args, name):
     from brax_amd.generalized import autotune
     autotune.set_launch(m, autotune.LANES, args.lanes)
   lanes = lib.bgx_model_get_launch(m.handle, 3)
-  kernel = "k_mtree" if lanes > 1 else "k_rollout"
+  kernel = {1: "k_rollout", 4: "k_star"}.get(lanes, "k_mtree")
   if lanes > 1:
-    # the multi-lane kernel's workgroup is one wavefront of 64 / lanes envs,
+    # a multi-lane kernel's workgroup is one wavefront of 64 / lanes envs,
     # and it keeps one contact row per candidate lane (no LDS tile)
     epw = 64 // lanes
   elif not args.no_tune:
@@ -384,7 +384,8 @@ def fwd_adjoint_leg(n, T, ckpt, warmup, tune=True, cpu=True, parts=0):
   autotune.set_launch(m, autotune.ADJOINT_PARTS, parts)
   epw = [64, 64]
   if tune:
-    epw[0] = autotune.tune_step(sys_, q0t, qd0t, acts0[:2], N_FRAMES)
+    if autotune.get_launch(m, autotune.LANES) == 1:
+      epw[0] = autotune.tune_step(sys_, q0t, qd0t, acts0[:2], N_FRAMES)
     # the backward pass over one checkpoint segment: a shorter window times
     # the launch overheads rather than the kernels
     epw[1] = autotune.tune_adjoint(sys_, q0t, qd0t, acts0[:ckpt], N_FRAMES)
@@ -626,9 +627,8 @@ def hetero_bench(args):
                  "parallelism": "none (1 GPU)"},
       "roofline": {"bound": "valu", "achieved": achieved, "peak": FP32_PEAK_TFLOPS,
                    "unit": "TFLOP/s", "frac": achieved / FP32_PEAK_TFLOPS,
-                   "traffic": measured_traffic("k_rollout", "hetero", n, K,
-                                               rel=f"profiles/hetero_{n}.md"),
-                   "traffic_source": f"profiles/hetero_{n}.md (rocprofv3 --pmc FETCH_SIZE, "
+                   "traffic": measured_traffic("k_star_batch", "hetero", n, K),
+                   "traffic_source": f"profiles/k_star_batch_hetero_{n}.md (rocprofv3 --pmc FETCH_SIZE, "
                                      "WRITE_SIZE of this command)",
                    "kernel_ms": kernel_ms,
                    "note": "op-count model: quadrupeds at R_a active rows, chains without rows",

@@ -721,7 +721,8 @@ int bgx_batch_create(int32_t n_models, const bgx_model* const* models,
     table_off[m] = tfloats;
     table_len[m] = ops->per_env ? (int64_t)n * size : size;
     tfloats += table_len[m];
-    const int per = ops->chain ? bgx::WAVE / bgx::chain_lanes(ops->dims[0]) : bgx::WAVE;
+    const int per = ops->chain ? bgx::WAVE / bgx::chain_lanes(ops->dims[0])
+                               : bgx::WAVE / std::max(ops->mlanes, 1);
     for (int i = 0; i < n; i += per) {
       bgx::BatchItem b{};
       b.m_off = table_off[m] + (ops->per_env ? (int64_t)i * size : 0);

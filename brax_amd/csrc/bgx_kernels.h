@@ -18,6 +18,7 @@
 #include "bgx_batch.h"
 #include "bgx_launch.h"
 #include "bgx_mtree.h"
+#include "bgx_star.h"
 #include "bgx_step.h"
 
 namespace bgx {
@@ -437,11 +438,21 @@ __global__ __launch_bounds__(WAVE) void k_adj_b(AdjLaunch a) {
   }
 }
 
+// whether the topology's batch items are a lane per leg (bgx_star.h)
+template <class T>
+constexpr bool star_tree() {
+  if constexpr (is_chain_kernel<T>()) return false;
+  else return star_ok<T>();
+}
+
 // a batch launch of the rollout kernel: a persistent grid of `grid`
 // one-wavefront workgroups (a.items set)
 template <class T>
 hipError_t launch_batch(const Launch& a, int grid, hipStream_t s) {
-  hipLaunchKernelGGL((k_rollout<T, true>), dim3((unsigned)grid), dim3(WAVE), 0, s, a);
+  if constexpr (star_tree<T>())
+    hipLaunchKernelGGL(k_star_batch<T>, dim3((unsigned)grid), dim3(WAVE), 0, s, a);
+  else
+    hipLaunchKernelGGL((k_rollout<T, true>), dim3((unsigned)grid), dim3(WAVE), 0, s, a);
   return hipGetLastError();
 }
 
@@ -449,9 +460,12 @@ hipError_t launch_batch(const Launch& a, int grid, hipStream_t s) {
 template <class T>
 int batch_blocks_per_cu() {
   int nb = 0;
-  if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&nb, k_rollout<T, true>, WAVE, 0) !=
-      hipSuccess)
-    return 1;
+  hipError_t e;
+  if constexpr (star_tree<T>())
+    e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&nb, k_star_batch<T>, WAVE, 0);
+  else
+    e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&nb, k_rollout<T, true>, WAVE, 0);
+  if (e != hipSuccess) return 1;
   return nb > 0 ? nb : 1;
 }
 
@@ -492,8 +506,12 @@ struct TopoOps {
 template <class T>
 struct Ops {
   static hipError_t init(const Launch& a, hipStream_t s) {
-    const int b = block_lanes(a.epw);
-    hipLaunchKernelGGL(k_init<T>, env_grid(a.n, b), dim3(b), 0, s, a);
+    if constexpr (star_ok<T>()) {
+      hipLaunchKernelGGL(k_star_init<T>, env_grid(a.n, STAR_ENVS), dim3(WAVE), 0, s, a);
+    } else {
+      const int b = block_lanes(a.epw);
+      hipLaunchKernelGGL(k_init<T>, env_grid(a.n, b), dim3(b), 0, s, a);
+    }
     return hipGetLastError();
   }
   template <class TT>
@@ -517,6 +535,16 @@ struct Ops {
         const hipError_t e = hipGetLastError();
         if (e != hipSuccess || !(a.x_pos || a.x_rot || a.xd_ang || a.xd_vel)) return e;
         return init(a, s);  // frames of the final state
+      }
+    }
+    if constexpr (star_ok<T>()) {
+      // a lane per leg, unless the caller chose one thread per env or one of
+      // that kernel's slot counts
+      if (a.lanes != 1 && a.kc == 0) {
+        const dim3 g = env_grid(a.n, STAR_ENVS);
+        hipLaunchKernelGGL(k_star<T>, dim3(g.x, a.n_seg > 1 ? (unsigned)a.n_seg : 1u),
+                           dim3(WAVE), 0, s, a);
+        return hipGetLastError();
       }
     }
     if constexpr (T::TILE1 > 0) {
@@ -572,7 +600,7 @@ struct Ops {
               nullptr};
     if constexpr (T::NCAND > 0) t.contacts = &contacts;
     t.frames_vjp = &frames_vjp;
-    t.mlanes = T::MLANE ? MTab<T>::G : 0;
+    t.mlanes = T::MLANE ? MTab<T>::G : (star_ok<T>() ? STAR_LEGS : 0);
     t.tiles[0] = T::KC, t.tiles[1] = T::TILE1, t.tiles[2] = T::TILE2;
     if constexpr (T::BATCH) t.batch = &launch_batch<T>, t.batch_occupancy = &batch_blocks_per_cu<T>;
     // the adjoint is compiled for topologies with a shared model table

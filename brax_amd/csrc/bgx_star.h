@@ -1,0 +1,1067 @@
+// Trees of one shape: a free root link with four equal legs (serial hinge
+// chains of K links), one lane per leg.
+//
+// One thread per env makes a substep of such a robot one dependent chain of
+// some 14,000 instructions without contacts, on a wavefront that has its SIMD
+// to itself (the tree's arrays fill the register file), so a call takes as
+// long for one robot as for 65,536.  Here an env is a quad of lanes: lane b
+// holds leg b, and every lane holds the root.  The legs' work goes on side by
+// side, the root's is repeated on the four lanes, and what the legs add to
+// the root (subtree forces, composite inertias, the factor's update, the
+// solver's dot products) are sums over the quad, two DPP additions each with
+// no LDS and no wait.  16 envs share a wavefront.
+//
+// The constrained products need no tree pass: with M = L^T L the rows
+// L^-T J^T of a lane's contacts and limits are formed once per substep (they
+// live on the lane's leg and the root: K + 6 numbers), and
+// A v = (L^-T J^T)^T (L^-T J^T) v + diag v is two dot products per row and
+// one quad sum of six.  Every candidate keeps a slot on its lane, so there is
+// no second path for many contacts; a slot that no lane of the wavefront
+// uses is skipped.  The step is the reference's (pipeline.py:64-94) as
+// bgx_step.h restates it.
+//
+// The four lanes of an env must agree bit for bit on the root and on every
+// decision: quad_sum adds commutatively and keeps the compiler from fusing
+// its additions with the lane's own products.
+#pragma once
+
+#include <hip/hip_runtime.h>
+
+#include "bgx_launch.h"
+#include "bgx_batch.h"
+#include "bgx_step.h"
+
+namespace bgx {
+
+constexpr int STAR_LEGS = 4;
+constexpr int STAR_ENVS = WAVE / STAR_LEGS;  // envs per wavefront
+
+// candidate index of the j-th candidate on leg b (-1: none), and of the j-th
+// on the root
+template <class T>
+constexpr int star_leg_cand(int b, int j) {
+  const int K = (T::L - 1) / STAR_LEGS;
+  for (int c = 0; c < T::NCAND; ++c) {
+    const int l = T::CAND_LINK[c];
+    if (l >= 1 + b * K && l < 1 + (b + 1) * K && j-- == 0) return c;
+  }
+  return -1;
+}
+template <class T>
+constexpr int star_root_cand(int j) {
+  for (int c = 0; c < T::NCAND; ++c)
+    if (T::CAND_LINK[c] == 0 && j-- == 0) return c;
+  return -1;
+}
+// the actuator / limit row of dof d, or -1
+template <class T>
+constexpr int star_act(int d) {
+  for (int u = 0; u < T::NU; ++u)
+    if (T::ACT_D[u] == d) return u;
+  return -1;
+}
+template <class T>
+constexpr bool star_lim(int d) {
+  for (int i = 0; i < T::NLIM; ++i)
+    if (T::LIM_D[i] == d) return true;
+  return false;
+}
+
+// whether topology T has this shape, leg by leg the same structure
+template <class T>
+constexpr bool star_ok() {
+  if (T::PER_ENV || T::PAIRS || !T::PLANE_Z || T::MLANE) return false;
+  if (T::L < 1 + STAR_LEGS || (T::L - 1) % STAR_LEGS != 0 || T::LTYPE[0] != 0) return false;
+  const int K = (T::L - 1) / STAR_LEGS;
+  if (K > 3 || T::PARENT[0] >= 0 || T::QADR[0] != 0 || T::DADR[0] != 0) return false;
+  for (int l = 1; l < T::L; ++l) {
+    const int k = (l - 1) % K, d = 5 + l;
+    if (T::LTYPE[l] != 1 || T::PARENT[l] != (k == 0 ? 0 : l - 1)) return false;
+    if (T::DADR[l] != d || T::QADR[l] != d + 1 || !T::DOF_HINGE[d]) return false;
+    if ((star_act<T>(d) >= 0) != (star_act<T>(6 + k) >= 0)) return false;
+    if (star_lim<T>(d) != star_lim<T>(6 + k)) return false;
+  }
+  for (int u = 0; u < T::NU; ++u) {
+    if (T::ACT_D[u] < 6 || T::ACT_Q[u] != T::ACT_D[u] + 1) return false;
+    if (star_act<T>(T::ACT_D[u]) != u) return false;  // one actuator per dof
+  }
+  for (int i = 0; i < T::NLIM; ++i)
+    if (T::LIM_D[i] < 6 || T::LIM_Q[i] != T::LIM_D[i] + 1) return false;
+  int per_leg = 0, on_root = 0;
+  while (star_leg_cand<T>(0, per_leg) >= 0) ++per_leg;
+  while (star_root_cand<T>(on_root) >= 0) ++on_root;
+  if (per_leg * STAR_LEGS + on_root != T::NCAND || per_leg > 4 || on_root > STAR_LEGS) return false;
+  for (int b = 0; b < STAR_LEGS; ++b) {
+    if (star_leg_cand<T>(b, per_leg) >= 0) return false;
+    for (int j = 0; j < per_leg; ++j) {
+      const int c0 = star_leg_cand<T>(0, j), c = star_leg_cand<T>(b, j);
+      if (c < 0 || T::CAND_KIND[c] != T::CAND_KIND[c0]) return false;
+      if (T::CAND_LINK[c] - b * K != T::CAND_LINK[c0]) return false;
+      // leg b's candidates at one distance from leg 0's
+      if (c - c0 != b * (star_leg_cand<T>(1, 0) - star_leg_cand<T>(0, 0))) return false;
+    }
+  }
+  // the root's candidates: one kind, consecutive
+  for (int j = 1; j < on_root; ++j) {
+    const int c = star_root_cand<T>(j), p = star_root_cand<T>(j - 1);
+    if (c < 1 || p != c - 1 || T::CAND_KIND[c] != T::CAND_KIND[c - 1]) return false;
+  }
+  return true;
+}
+
+template <class T>
+struct Star {
+  static constexpr int K = (T::L - 1) / STAR_LEGS;
+  static constexpr int NCL = [] {
+    int j = 0;
+    while (star_leg_cand<T>(0, j) >= 0) ++j;
+    return j;
+  }();
+  static constexpr int NCR = T::NCAND - STAR_LEGS * NCL;  // on the root, lane j holds the j-th
+  static constexpr int S = NCL + (NCR > 0 ? 1 : 0);       // slots of a lane
+  static constexpr int SN = S > 0 ? S : 1;
+  static constexpr int CSTEP = NCL > 0 ? star_leg_cand<T>(1, 0) - star_leg_cand<T>(0, 0) : 0;
+  // last leg link whose dofs move slot s's link (-1: the root)
+  static constexpr int link(int s) {
+    return s < NCL ? T::CAND_LINK[star_leg_cand<T>(0, s)] - 1 : -1;
+  }
+  static constexpr int cand0(int s) {
+    return s < NCL ? star_leg_cand<T>(0, s) : star_root_cand<T>(0);
+  }
+};
+
+// the sum of x over the env's quad, the same bits on its four lanes; every
+// lane of the quad must be active
+BGX_D float quad_sum(float x) {
+#pragma clang fp contract(off)
+  asm("" : "+v"(x));
+  const float y =
+      x + __builtin_bit_cast(float, __builtin_amdgcn_mov_dpp(__builtin_bit_cast(int, x), 0xB1,
+                                                             0xf, 0xf, true));
+  return y + __builtin_bit_cast(float, __builtin_amdgcn_mov_dpp(__builtin_bit_cast(int, y), 0x4E,
+                                                                0xf, 0xf, true));
+}
+BGX_D V3 quad_sum(V3 v) { return V3{quad_sum(v.x), quad_sum(v.y), quad_sum(v.z)}; }
+// the lanes of this lane's quad for which p holds
+BGX_D unsigned quad_ballot(bool p) {
+  return (unsigned)(__ballot(p) >> (threadIdx.x & (WAVE - STAR_LEGS))) & 0xfu;
+}
+template <class X>
+BGX_D X by_leg(int b, X x0, X x1, X x2, X x3) {
+  const X lo = (b & 1) ? x1 : x0, hi = (b & 1) ? x3 : x2;
+  return (b & 2) ? hi : lo;
+}
+// the actuator of leg b's k-th hinge
+template <class T>
+BGX_D int star_act_of_leg(int b, int k) {
+  constexpr int K = Star<T>::K;
+  return by_leg(b, star_act<T>(6 + k), star_act<T>(6 + K + k), star_act<T>(6 + 2 * K + k),
+                star_act<T>(6 + 3 * K + k));
+}
+
+template <class T>
+struct StarState {
+  static constexpr int K = Star<T>::K;
+  float rq[7], rv[6];  // root, the same on the four lanes
+  float q[K], qd[K];   // this lane's leg
+};
+
+// the state from / to an env's rows; the root's entries are spread over the
+// quad, so that a wavefront's stores cover whole rows
+template <class T>
+BGX_D void star_load(StarState<T>& s, int b, const float* qp, const float* qdp) {
+  constexpr int K = Star<T>::K;
+#pragma unroll
+  for (int k = 0; k < 7; ++k) s.rq[k] = qp[k];
+#pragma unroll
+  for (int k = 0; k < 6; ++k) s.rv[k] = qdp[k];
+#pragma unroll
+  for (int k = 0; k < K; ++k) s.q[k] = qp[7 + b * K + k], s.qd[k] = qdp[6 + b * K + k];
+}
+template <class T>
+BGX_D void star_store_q(const StarState<T>& s, int b, float* qp) {
+  constexpr int K = Star<T>::K;
+  qp[b] = by_leg(b, s.rq[0], s.rq[1], s.rq[2], s.rq[3]);
+  if (b < 3) qp[4 + b] = by_leg(b, s.rq[4], s.rq[5], s.rq[6], 0.f);
+#pragma unroll
+  for (int k = 0; k < K; ++k) qp[7 + b * K + k] = s.q[k];
+}
+template <class T>
+BGX_D void star_store_qd(const StarState<T>& s, int b, float* qdp) {
+  constexpr int K = Star<T>::K;
+  qdp[b] = by_leg(b, s.rv[0], s.rv[1], s.rv[2], s.rv[3]);
+  if (b < 2) qdp[4 + b] = by_leg(b, s.rv[4], s.rv[5], 0.f, 0.f);
+#pragma unroll
+  for (int k = 0; k < K; ++k) qdp[6 + b * K + k] = s.qd[k];
+}
+
+// world frames of the root and of this lane's leg (kinematics.py:31-108);
+// XD: also the frames' velocities
+template <class T, bool XD>
+BGX_D void star_frames(const float* ml, int b, const StarState<T>& s, V3& xp0, Q4& xr0, V3* xp,
+                       Q4* xr, V3* xa0, V3* xa, V3* xv) {
+  constexpr int K = Star<T>::K;
+  const float* lk = ml + T::OFF_LINK;
+  {
+    V3 p = v3(s.rq[0], s.rq[1], s.rq[2]);
+    const Q4 r{s.rq[3], s.rq[4], s.rq[5], s.rq[6]};
+    const V3 jpos = ldv3(lk + LK_JPOS);
+    p = (p + jpos) - rotate(jpos, r);
+    const Q4 trot = ldq4(lk + LK_TROT);
+    xp0 = ldv3(lk + LK_TPOS) + rotate(p, trot);
+    xr0 = qmul(trot, r);
+  }
+  if constexpr (XD) *xa0 = rotate(v3(s.rv[3], s.rv[4], s.rv[5]), xr0);
+  lk += LINK_STRIDE * (1 + b * K);
+  const float* df = ml + T::OFF_DOF + DOF_STRIDE * (6 + b * K);
+#pragma unroll
+  for (int k = 0; k < K; ++k, lk += LINK_STRIDE, df += DOF_STRIDE) {
+    const V3 ang = ldv3(df + DF_ANG);
+    const Q4 rk = qnormalize(qrot_axis(ang, s.q[k]));
+    const V3 jpos = ldv3(lk + LK_JPOS);
+    const Q4 trot = ldq4(lk + LK_TROT);
+    const V3 p = ldv3(lk + LK_TPOS) + rotate(jpos - rotate(jpos, rk), trot);
+    const V3 pp = k == 0 ? xp0 : xp[k - 1];
+    const Q4 pr = k == 0 ? xr0 : xr[k - 1];
+    xp[k] = pp + rotate(p, pr);
+    xr[k] = qmul(pr, qmul(trot, rk));
+    if constexpr (XD) {
+      const V3 pa = k == 0 ? *xa0 : xa[k - 1];
+      const V3 pv = k == 0 ? v3(s.rv[0], s.rv[1], s.rv[2]) : xv[k - 1];
+      xv[k] = pv + cross(pa, xp[k] - pp);
+      xa[k] = pa + rotate(ang * s.qd[k], xr[k]);
+    }
+  }
+  xr0 = qnormalize(xr0);
+#pragma unroll
+  for (int k = 0; k < K; ++k) xr[k] = qnormalize(xr[k]);
+}
+
+// mass-weighted COM offset and rotational inertia of one link about rc
+// (dynamics.py:44-55)
+BGX_D void star_inertia(const float* lk, V3 xp, Q4 xr, V3 rc, V3& cc, Sym3& ci) {
+  const V3 p = (xp + rotate(ldv3(lk + LK_IPOS), xr)) - rc;
+  const float m = lk[LK_MASS];
+  float R[3][3], RI[3][3];
+  quat_to_3x3(qmul(xr, ldq4(lk + LK_IROT)), R);
+  const Sym3 I0 = ldsym(lk + LK_I);
+#pragma unroll
+  for (int i = 0; i < 3; ++i) {
+    const V3 c = symmul(I0, V3{R[i][0], R[i][1], R[i][2]});
+    RI[i][0] = c.x, RI[i][1] = c.y, RI[i][2] = c.z;
+  }
+  auto rir = [&](int i, int j) {
+    return RI[i][0] * R[j][0] + RI[i][1] * R[j][1] + RI[i][2] * R[j][2];
+  };
+  const float pp = dot(p, p);
+  ci = Sym3{rir(0, 0) + (pp - p.x * p.x) * m, rir(1, 1) + (pp - p.y * p.y) * m,
+            rir(2, 2) + (pp - p.z * p.z) * m, rir(0, 1) - p.x * p.y * m,
+            rir(0, 2) - p.x * p.z * m, rir(1, 2) - p.y * p.z * m};
+  cc = p * m;
+}
+
+// M = L^T L of the env: this leg's block and its columns at the root, and
+// the root's block (the same on the four lanes); inv: 1 / diagonal of L
+template <int K>
+struct StarFactor {
+  float leg[K][K], col[K][6], root[6][6], inv[K], inv0[6];
+
+  // z = L^-T z, a vector that lives on this leg and the root alone
+  BGX_D void lt_own(float* z, float* zr) const {
+#pragma unroll
+    for (int k = K - 1; k >= 0; --k) {
+      z[k] *= inv[k];
+#pragma unroll
+      for (int j = 0; j < k; ++j) z[j] -= leg[k][j] * z[k];
+#pragma unroll
+      for (int j = 0; j < 6; ++j) zr[j] -= col[k][j] * z[k];
+    }
+    lt_root(zr);
+  }
+  BGX_D void lt_root(float* zr) const {
+#pragma unroll
+    for (int i = 5; i >= 0; --i) {
+      zr[i] *= inv0[i];
+#pragma unroll
+      for (int j = 0; j < i; ++j) zr[j] -= root[i][j] * zr[i];
+    }
+  }
+  // z = L^-T z of a whole env's vector
+  BGX_D void lt(float* z, float* zr) const {
+    float p[6] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int k = K - 1; k >= 0; --k) {
+      z[k] *= inv[k];
+#pragma unroll
+      for (int j = 0; j < k; ++j) z[j] -= leg[k][j] * z[k];
+#pragma unroll
+      for (int j = 0; j < 6; ++j) p[j] += col[k][j] * z[k];
+    }
+#pragma unroll
+    for (int j = 0; j < 6; ++j) zr[j] -= quad_sum(p[j]);
+    lt_root(zr);
+  }
+  // z = L^-1 z of a whole env's vector
+  BGX_D void l(float* z, float* zr) const {
+#pragma unroll
+    for (int i = 0; i < 6; ++i) {
+#pragma unroll
+      for (int j = 0; j < i; ++j) zr[i] -= root[i][j] * zr[j];
+      zr[i] *= inv0[i];
+    }
+#pragma unroll
+    for (int k = 0; k < K; ++k) {
+#pragma unroll
+      for (int j = 0; j < 6; ++j) z[k] -= col[k][j] * zr[j];
+#pragma unroll
+      for (int j = 0; j < k; ++j) z[k] -= leg[k][j] * z[j];
+      z[k] *= inv[k];
+    }
+  }
+};
+
+// The contact rows of a lane: slot i's row x = L^-T J^T along n, mu t1 or
+// mu t2, K + 6 numbers (leg, then root).  Up to two slots stay in registers;
+// more would push the solver's vectors into accumulation registers, a move
+// for every use, so they live in LDS: float4 q of a row at
+// base[(q WAVE + lane) 4], read without bank conflicts.
+template <class T>
+struct StarRows {
+  static constexpr int K = Star<T>::K, W = (K + 6 + 3) / 4 * 4, Q = W / 4;
+  static constexpr bool LDS = Star<T>::S > 2;
+  static constexpr int FLOATS = LDS ? Star<T>::S * 3 * W * WAVE : 0;
+  float4* base;
+  float r[LDS ? 1 : Star<T>::SN][3][W];
+  BGX_D void put(int i, int x, const float* v) {
+    if constexpr (LDS) {
+#pragma unroll
+      for (int q = 0; q < Q; ++q)
+        base[((i * 3 + x) * Q + q) * WAVE] =
+            float4{v[4 * q], v[4 * q + 1], v[4 * q + 2], v[4 * q + 3]};
+    } else {
+#pragma unroll
+      for (int k = 0; k < W; ++k) r[i][x][k] = v[k];
+    }
+  }
+  BGX_D void get(int i, int x, float* v) const {
+    if constexpr (LDS) {
+#pragma unroll
+      for (int q = 0; q < Q; ++q) {
+        const float4 f = base[((i * 3 + x) * Q + q) * WAVE];
+        v[4 * q] = f.x, v[4 * q + 1] = f.y, v[4 * q + 2] = f.z, v[4 * q + 3] = f.w;
+      }
+    } else {
+#pragma unroll
+      for (int k = 0; k < W; ++k) v[k] = r[i][x][k];
+    }
+  }
+};
+
+// LDS of a wavefront (floats): the model table, then the contact rows
+template <class T>
+constexpr int star_table_floats() { return (T::SIZE + 3) / 4 * 4; }
+template <class T>
+constexpr int star_lds_floats() { return star_table_floats<T>() + StarRows<T>::FLOATS; }
+
+// one substep (pipeline.step, pipeline.py:64-94).  ml: the model table in
+// LDS; probe (or null): the env's probe row.  Returns the active contacts.
+template <class T>
+BGX_D int star_substep(float* ml, int b, StarState<T>& s, const float* act,
+                       float* probe) {
+  using SR = Star<T>;
+  constexpr int K = SR::K, S = SR::S, SN = SR::SN, NV = T::NV;
+  const float* lk0 = ml + T::OFF_LINK;
+  const float* lkb = lk0 + LINK_STRIDE * (1 + b * K);
+  const float* df0 = ml + T::OFF_DOF;
+  const float* dfb = df0 + DOF_STRIDE * (6 + b * K);
+
+  V3 xp0, xp[K];
+  Q4 xr0, xr[K];
+  star_frames<T, false>(ml, b, s, xp0, xr0, xp, xr, nullptr, nullptr, nullptr);
+
+  // ---- root COM (dynamics.py:37-43), cinr (:44-55)
+  const float m0 = lk0[LK_MASS];
+  V3 rc;
+  {
+    V3 sm = v3zero();
+    float ms = 0.f;
+#pragma unroll
+    for (int k = 0; k < K; ++k) {
+      const float* lk = lkb + LINK_STRIDE * k;
+      sm = sm + (xp[k] + rotate(ldv3(lk + LK_IPOS), xr[k])) * lk[LK_MASS];
+      ms = ms + lk[LK_MASS];
+    }
+    sm = (xp0 + rotate(ldv3(lk0 + LK_IPOS), xr0)) * m0 + quad_sum(sm);
+    const float ims = rcp(m0 + quad_sum(ms));
+    rc = V3{sm.x * ims, sm.y * ims, sm.z * ims};
+  }
+  V3 cc0, cc[K];
+  Sym3 ci0, ci[K];
+  float km[K];
+  star_inertia(lk0, xp0, xr0, rc, cc0, ci0);
+#pragma unroll
+  for (int k = 0; k < K; ++k) {
+    star_inertia(lkb + LINK_STRIDE * k, xp[k], xr[k], rc, cc[k], ci[k]);
+    km[k] = lkb[LINK_STRIDE * k + LK_MASS];
+  }
+
+  // ---- cdof (dynamics.py:56-89): the root's translations are the world's
+  // axes, its rotations (ra, rv); the leg's hinges (ca, cv)
+  V3 ra[3], rv[3], ca[K], cv[K];
+  {
+    const Q4 jr = qmul(xr0, ldq4(lk0 + LK_TROT));
+    const V3 jp = (xp0 + rotate(ldv3(lk0 + LK_TPOS), xr0)) + rotate(ldv3(lk0 + LK_JPOS), jr);
+    const V3 off = rc - jp;
+#pragma unroll
+    for (int k = 0; k < 3; ++k) {
+      ra[k] = rotate(unit3(k), jr);
+      rv[k] = cross(ra[k], off);
+    }
+  }
+#pragma unroll
+  for (int k = 0; k < K; ++k) {
+    const float* lk = lkb + LINK_STRIDE * k;
+    const V3 pp = k == 0 ? xp0 : xp[k - 1];
+    const Q4 pr = k == 0 ? xr0 : xr[k - 1];
+    const Q4 jr = qmul(pr, ldq4(lk + LK_TROT));
+    const V3 jp = (pp + rotate(ldv3(lk + LK_TPOS), pr)) + rotate(ldv3(lk + LK_JPOS), jr);
+    ca[k] = rotate(ldv3(dfb + DOF_STRIDE * k + DF_ANG), jr);
+    cv[k] = cross(ca[k], rc - jp);
+  }
+
+  // ---- link velocities (dynamics.py:90-103)
+  const V3 rlin = v3(s.rv[0], s.rv[1], s.rv[2]);
+  const V3 va0 = ra[0] * s.rv[3] + ra[1] * s.rv[4] + ra[2] * s.rv[5];
+  const V3 vv0 = rlin + (rv[0] * s.rv[3] + rv[1] * s.rv[4] + rv[2] * s.rv[5]);
+  V3 va[K], vv[K];
+#pragma unroll
+  for (int k = 0; k < K; ++k) {
+    va[k] = (k == 0 ? va0 : va[k - 1]) + ca[k] * s.qd[k];
+    vv[k] = (k == 0 ? vv0 : vv[k - 1]) + cv[k] * s.qd[k];
+  }
+
+  // ---- RNEA bias (dynamics.py:105-184), passive and actuator forces
+  // (:187-236, actuator.py:23-57)
+  float z[K], zr[6];  // qf_smooth
+  {
+    const V3 acc0 = cross(rlin, va0) - ldv3(ml + H_GRAVITY);  // linear; no angular part
+    V3 f2a, f2v, f3a, f3v;
+    inertia_mul(cc0, ci0, m0, va0, vv0, f2a, f2v);
+    cross_force(va0, vv0, f2a, f2v, f3a, f3v);
+    const V3 fa0 = cross(cc0, acc0) + f3a, fv0 = acc0 * m0 + f3v;
+    V3 aa = v3zero(), av = acc0, fa[K], fv[K];
+#pragma unroll
+    for (int k = 0; k < K; ++k) {
+      V3 oa, ov, f1a, f1v;
+      cross_motion(k == 0 ? va0 : va[k - 1], k == 0 ? vv0 : vv[k - 1], ca[k], cv[k], oa, ov);
+      aa = aa + oa * s.qd[k], av = av + ov * s.qd[k];
+      inertia_mul(cc[k], ci[k], km[k], aa, av, f1a, f1v);
+      inertia_mul(cc[k], ci[k], km[k], va[k], vv[k], f2a, f2v);
+      cross_force(va[k], vv[k], f2a, f2v, f3a, f3v);
+      fa[k] = f1a + f3a, fv[k] = f1v + f3v;
+    }
+#pragma unroll
+    for (int k = K - 1; k >= 0; --k) {
+      if (k + 1 < K) fa[k] = fa[k] + fa[k + 1], fv[k] = fv[k] + fv[k + 1];
+      const float* df = dfb + DOF_STRIDE * k;
+      float p = -df[DF_DAMPING] * s.qd[k];
+      p = -s.q[k] * df[DF_STIFFNESS] + p;
+      z[k] = p - (dot(cv[k], fv[k]) + dot(ca[k], fa[k]));
+      if (star_act<T>(6 + k) >= 0) {
+        const float* ac = ml + T::OFF_ACT + star_act_of_leg<T>(b, k) * ACT_STRIDE;
+        const float ctl = clipf(act[k], ac[AC_CTRL_LO], ac[AC_CTRL_HI]);
+        const float bias = ac[AC_GEAR] * (s.q[k] * ac[AC_BIAS_Q] + s.qd[k] * ac[AC_BIAS_QD]);
+        z[k] += clipf(ac[AC_GAIN] * ctl + bias, ac[AC_FORCE_LO], ac[AC_FORCE_HI]) * ac[AC_GEAR];
+      }
+    }
+    const V3 Fa = fa0 + quad_sum(fa[0]), Fv = fv0 + quad_sum(fv[0]);
+    zr[0] = Fv.x, zr[1] = Fv.y, zr[2] = Fv.z;
+#pragma unroll
+    for (int k = 0; k < 3; ++k) zr[3 + k] = dot(rv[k], Fv) + dot(ra[k], Fa);
+#pragma unroll
+    for (int k = 0; k < 6; ++k) zr[k] = -df0[DOF_STRIDE * k + DF_DAMPING] * s.rv[k] - zr[k];
+  }
+  if (probe) {
+#pragma unroll
+    for (int k = 0; k < K; ++k) probe[6 + b * K + k] = z[k];
+    if (b == 0)
+#pragma unroll
+      for (int k = 0; k < 6; ++k) probe[k] = zr[k];
+  }
+
+  // ---- mass.matrix (mass.py:27-83) and its factor, leaves first
+  StarFactor<K> F;
+  {
+#pragma unroll
+    for (int k = K - 1; k > 0; --k) {
+      cc[k - 1] = cc[k - 1] + cc[k];
+      ci[k - 1] = symadd(ci[k - 1], ci[k]);
+      km[k - 1] = km[k - 1] + km[k];
+    }
+    float up[6][6];
+#pragma unroll
+    for (int k = 0; k < K; ++k) {
+      V3 fa, fv;
+      inertia_mul(cc[k], ci[k], km[k], ca[k], cv[k], fa, fv);
+      F.leg[k][k] = dot(cv[k], fv) + dot(ca[k], fa) + dfb[DOF_STRIDE * k + DF_ARMATURE];
+#pragma unroll
+      for (int j = 0; j < k; ++j) F.leg[k][j] = dot(cv[j], fv) + dot(ca[j], fa);
+      F.col[k][0] = fv.x, F.col[k][1] = fv.y, F.col[k][2] = fv.z;
+#pragma unroll
+      for (int j = 0; j < 3; ++j) F.col[k][3 + j] = dot(rv[j], fv) + dot(ra[j], fa);
+    }
+#pragma unroll
+    for (int k = K - 1; k >= 0; --k) {
+      const float lkk = fsqrt(F.leg[k][k]);
+      F.inv[k] = rcp(lkk);
+#pragma unroll
+      for (int j = 0; j < k; ++j) F.leg[k][j] *= F.inv[k];
+#pragma unroll
+      for (int j = 0; j < 6; ++j) F.col[k][j] *= F.inv[k];
+#pragma unroll
+      for (int i = 0; i < k; ++i) {
+        const float a = F.leg[k][i];
+#pragma unroll
+        for (int j = 0; j <= i; ++j) F.leg[i][j] -= a * F.leg[k][j];
+#pragma unroll
+        for (int j = 0; j < 6; ++j) F.col[i][j] -= a * F.col[k][j];
+      }
+#pragma unroll
+      for (int i = 0; i < 6; ++i)
+#pragma unroll
+        for (int j = 0; j <= i; ++j)
+          up[i][j] = (k == K - 1 ? 0.f : up[i][j]) + F.col[k][i] * F.col[k][j];
+    }
+    const V3 tc = cc0 + quad_sum(cc[0]);
+    const Sym3 ti{ci0.xx + quad_sum(ci[0].xx), ci0.yy + quad_sum(ci[0].yy),
+                  ci0.zz + quad_sum(ci[0].zz), ci0.xy + quad_sum(ci[0].xy),
+                  ci0.xz + quad_sum(ci[0].xz), ci0.yz + quad_sum(ci[0].yz)};
+    const float tm = m0 + quad_sum(km[0]);
+#pragma unroll
+    for (int i = 0; i < 3; ++i) {
+      V3 fa, fv;
+      inertia_mul(tc, ti, tm, ra[i], rv[i], fa, fv);
+      F.root[3 + i][0] = fv.x, F.root[3 + i][1] = fv.y, F.root[3 + i][2] = fv.z;
+#pragma unroll
+      for (int j = 0; j <= i; ++j) F.root[3 + i][3 + j] = dot(rv[j], fv) + dot(ra[j], fa);
+#pragma unroll
+      for (int j = 0; j <= i; ++j) F.root[i][j] = j == i ? tm : 0.f;
+    }
+#pragma unroll
+    for (int i = 0; i < 6; ++i) F.root[i][i] += df0[DOF_STRIDE * i + DF_ARMATURE];
+#pragma unroll
+    for (int i = 0; i < 6; ++i)
+#pragma unroll
+      for (int j = 0; j <= i; ++j) F.root[i][j] -= quad_sum(up[i][j]);
+#pragma unroll
+    for (int k = 5; k >= 0; --k) {
+      F.inv0[k] = rcp(fsqrt(F.root[k][k]));
+#pragma unroll
+      for (int j = 0; j < k; ++j) F.root[k][j] *= F.inv0[k];
+#pragma unroll
+      for (int i = 0; i < k; ++i) {
+        const float a = F.root[k][i];
+#pragma unroll
+        for (int j = 0; j <= i; ++j) F.root[i][j] -= a * F.root[k][j];
+      }
+    }
+  }
+
+  // ---- w = L^-T qf_smooth; the unconstrained acceleration is L^-1 w
+  float w[K], wr[6];
+#pragma unroll
+  for (int k = 0; k < K; ++k) w[k] = z[k];
+#pragma unroll
+  for (int k = 0; k < 6; ++k) wr[k] = zr[k];
+  F.lt(w, wr);
+
+  // ---- contact rows (contact.py + MJX plane collisions, constraint.py):
+  // slot s has three rows of L^-T J^T, along n, mu t1 and mu t2 (its pyramid
+  // rows are n + mu t, n - mu t), on the leg jl and the root jr
+  using SRows = StarRows<T>;
+  SRows J;
+  J.base = (float4*)(ml + star_table_floats<T>()) + threadIdx.x % WAVE;
+  float diag[SN], sb[SN][4];
+  bool on[SN];  // slots that any lane of the wavefront uses
+  bool active[SN];
+  int n_c = 0;
+#pragma unroll
+  for (int i = 0; i < S; ++i) {
+    constexpr int NCL = SR::NCL;
+    const bool leg = i < NCL;
+    const int kk = SR::link(i);
+    const int c0 = SR::cand0(i);
+    const bool held = leg || b < SR::NCR;
+    const float* cd = ml + T::OFF_CAND +
+                      CAND_STRIDE * (c0 + (leg ? b * SR::CSTEP : (held ? b : 0)));
+    const V3 xpl = leg ? xp[kk >= 0 ? kk : 0] : xp0;
+    const Q4 xrl = leg ? xr[kk >= 0 ? kk : 0] : xr0;
+    V3 ctr = xpl + rotate(ldv3(cd + CD_GPOS), xrl);
+    V3 axis = v3zero();
+    if (T::CAND_KIND[c0] == KIND_CAPSULE) {
+      axis = quat_zaxis(qmul(xrl, ldq4(cd + CD_GQUAT)));
+      ctr = ctr + axis * (cd[CD_HALFLEN] * cd[CD_SIGN]);
+    }
+    const float radius = cd[CD_RADIUS];
+    const float dist = (ctr.z - cd[CD_PPOS + 2]) - radius;
+    active[i] = held && dist < 0.f;
+    on[i] = __ballot(active[i]) != 0ull;
+    n_c += __builtin_popcount(quad_ballot(active[i]));
+    diag[i] = 0.f;
+#pragma unroll
+    for (int k = 0; k < 4; ++k) sb[i][k] = 0.f;
+    if (on[i]) {
+      float j[3][SRows::W];  // this slot's rows
+#pragma unroll
+      for (int x = 0; x < 3; ++x)
+#pragma unroll
+        for (int k = 0; k < SRows::W; ++k) j[x][k] = 0.f;
+      V3 t1 = ldv3(cd + CD_T1);
+      if (T::CAND_KIND[c0] == KIND_CAPSULE) {
+        // along the capsule where it lies, y where it stands
+        float bn;
+        const V3 bt = vnormalize(v3(axis.x, axis.y, 0.f), &bn);
+        t1 = bn < 0.5f ? v3(0.f, 1.f, 0.f) : bt;
+      }
+      const float mu = cd[CD_MU], tw = cd[CD_TW];
+      const float* im = cd + CD_IMP;
+      const float imp = impedance(im, dist);
+      const V3 r = v3(ctr.x, ctr.y, ctr.z - (radius + 0.5f * dist)) - rc;
+      const float az = active[i] ? 1.f : 0.f;
+      const float ax = active[i] ? t1.x * mu : 0.f, ay = active[i] ? t1.y * mu : 0.f;
+      diag[i] = active[i] ? (tw + mu * mu * tw) * (2.f * mu * mu * imp_ratio(imp)) : 0.f;
+      auto rows = [&](V3 v, float& e0, float& e1, float& e2) {
+        e0 = az * v.z;
+        e1 = ax * v.x + ay * v.y;
+        e2 = ax * v.y - ay * v.x;
+      };
+#pragma unroll
+      for (int k = 0; k < K; ++k)
+        if (k <= kk) rows(cv[k] + cross(ca[k], r), j[0][k], j[1][k], j[2][k]);
+#pragma unroll
+      for (int k = 0; k < 3; ++k) {
+        rows(unit3(k), j[0][K + k], j[1][K + k], j[2][K + k]);
+        rows(rv[k] + cross(ra[k], r), j[0][K + 3 + k], j[1][K + 3 + k], j[2][K + 3 + k]);
+      }
+      // velocity of the contact point at qd
+      const V3 ka = leg ? va[kk >= 0 ? kk : 0] : va0, kv = leg ? vv[kk >= 0 ? kk : 0] : vv0;
+      float q0, q1, q2, e[3];
+      rows(kv + cross(ka, r), q0, q1, q2);
+#pragma unroll
+      for (int x = 0; x < 3; ++x) {
+        F.lt_own(j[x], j[x] + K);
+        J.put(i, x, j[x]);
+        e[x] = 0.f;
+#pragma unroll
+        for (int k = 0; k < K; ++k) e[x] += j[x][k] * w[k];
+#pragma unroll
+        for (int k = 0; k < 6; ++k) e[x] += j[x][K + k] * wr[k];
+      }
+      const float kt = active[i] ? im[IM_K] * imp * dist : 0.f, bq = im[IM_B];
+      sb[i][0] = (e[0] + e[1]) + (bq * (q0 + q1) + kt);
+      sb[i][1] = (e[0] - e[1]) + (bq * (q0 - q1) + kt);
+      sb[i][2] = (e[0] + e[2]) + (bq * (q0 + q2) + kt);
+      sb[i][3] = (e[0] - e[2]) + (bq * (q0 - q2) + kt);
+    }
+  }
+
+  // ---- u = M^-1 qf_smooth
+  float u[K], ur[6];
+#pragma unroll
+  for (int k = 0; k < K; ++k) u[k] = w[k];
+#pragma unroll
+  for (int k = 0; k < 6; ++k) ur[k] = wr[k];
+  F.l(u, ur);
+
+  // ---- limit rows (constraint.py:101-132): side times a row of L^-T
+  float ll[K][K], lr[K][6], ldiag[K], lb[K];
+  bool act_l[K];
+  bool any_l = false;
+#pragma unroll
+  for (int k = 0; k < K; ++k) {
+    act_l[k] = false, ldiag[k] = 0.f, lb[k] = 0.f;
+    if (!star_lim<T>(6 + k)) continue;
+    const float* df = dfb + DOF_STRIDE * k;
+    const float pmin = s.q[k] - df[DF_LO], pmax = df[DF_HI] - s.q[k];
+    const float pos = fminf(fminf(pmin, pmax), 0.f);
+    act_l[k] = pos < 0.f;
+    const float side = act_l[k] ? (pmin < pmax ? 1.f : -1.f) : 0.f;
+    const float* im = df + DF_IMP;
+    const float imp = impedance(im, pos);
+    const float aref = act_l[k] ? (-im[IM_B] * (side * s.qd[k]) - im[IM_K] * imp * pos) : 0.f;
+    ldiag[k] = act_l[k] ? df[DF_INVWEIGHT] * imp_ratio(imp) : 0.f;
+    lb[k] = side * u[k] - aref;
+#pragma unroll
+    for (int j = 0; j < K; ++j) ll[k][j] = j == k ? side : 0.f;
+#pragma unroll
+    for (int j = 0; j < 6; ++j) lr[k][j] = 0.f;
+    any_l = any_l || act_l[k];
+  }
+  const bool on_l = __ballot(any_l) != 0ull;
+  if (on_l) {
+#pragma unroll
+    for (int k = 0; k < K; ++k)
+      if (star_lim<T>(6 + k)) F.lt_own(ll[k], lr[k]);
+  }
+
+  bool mine = any_l;
+#pragma unroll
+  for (int i = 0; i < S; ++i) mine = mine || active[i];
+  const bool has_rows = quad_ballot(mine) != 0u;
+  int iters = 0, trials = 0;
+  if (__ballot(has_rows) != 0ull) {
+    // ---- jaxopt.ProjectedGradient: FISTA + backtracking line search from 0;
+    // an env's control is the same on its four lanes
+    float X[SN][4], Y[SN][4], G[SN][4], R[SN][4];
+    float xl[K], yl[K], gl[K], rl[K];
+#pragma unroll
+    for (int i = 0; i < SN; ++i)
+#pragma unroll
+      for (int k = 0; k < 4; ++k) X[i][k] = Y[i][k] = G[i][k] = R[i][k] = 0.f;
+#pragma unroll
+    for (int k = 0; k < K; ++k) xl[k] = yl[k] = gl[k] = rl[k] = 0.f;
+    // t = (L^-T J^T) in
+    auto gather = [&](auto in, auto in_l, float* t, float* tr) {
+      float p[6] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int k = 0; k < K; ++k) t[k] = 0.f;
+#pragma unroll
+      for (int i = 0; i < S; ++i) {
+        if (on[i]) {
+          const float v0 = in(i, 0), v1 = in(i, 1), v2 = in(i, 2), v3_ = in(i, 3);
+          const float a[3] = {(v0 + v1) + (v2 + v3_), v0 - v1, v2 - v3_};
+#pragma unroll
+          for (int x = 0; x < 3; ++x) {
+            float j[SRows::W];
+            J.get(i, x, j);
+#pragma unroll
+            for (int k = 0; k < K; ++k)
+              if (k <= SR::link(i)) t[k] += a[x] * j[k];
+#pragma unroll
+            for (int k = 0; k < 6; ++k) p[k] += a[x] * j[K + k];
+          }
+        }
+      }
+      if (on_l) {
+#pragma unroll
+        for (int k = 0; k < K; ++k) {
+          if (!star_lim<T>(6 + k)) continue;
+          const float v = in_l(k);
+#pragma unroll
+          for (int j = 0; j <= k; ++j) t[j] += v * ll[k][j];
+#pragma unroll
+          for (int j = 0; j < 6; ++j) p[j] += v * lr[k][j];
+        }
+      }
+#pragma unroll
+      for (int k = 0; k < 6; ++k) tr[k] = quad_sum(p[k]);
+    };
+    // out = A in
+    auto apply = [&](auto in, auto in_l, auto out, auto out_l) {
+      float t[K], tr[6];
+      gather(in, in_l, t, tr);
+#pragma unroll
+      for (int i = 0; i < S; ++i) {
+        if (on[i]) {
+          float e[3];
+#pragma unroll
+          for (int x = 0; x < 3; ++x) {
+            float j[SRows::W];
+            J.get(i, x, j);
+            e[x] = 0.f;
+#pragma unroll
+            for (int k = 0; k < 6; ++k) e[x] += j[K + k] * tr[k];
+#pragma unroll
+            for (int k = 0; k < K; ++k)
+              if (k <= SR::link(i)) e[x] += j[k] * t[k];
+          }
+          out(i, 0, e[0] + e[1] + diag[i] * in(i, 0));
+          out(i, 1, e[0] - e[1] + diag[i] * in(i, 1));
+          out(i, 2, e[0] + e[2] + diag[i] * in(i, 2));
+          out(i, 3, e[0] - e[2] + diag[i] * in(i, 3));
+        }
+      }
+      if (on_l) {
+#pragma unroll
+        for (int k = 0; k < K; ++k) {
+          if (!star_lim<T>(6 + k)) continue;
+          float e = 0.f;
+#pragma unroll
+          for (int j = 0; j < 6; ++j) e += lr[k][j] * tr[j];
+#pragma unroll
+          for (int j = 0; j <= k; ++j) e += ll[k][j] * t[j];
+          out_l(k, e + ldiag[k] * in_l(k));
+        }
+      }
+    };
+    const int maxiter = (int)ml[H_MAXITER], maxls = (int)ml[H_MAXLS];
+    const float tol = ml[H_TOL], lseps = ml[H_LSEPS];
+    float tk = 1.f, eta = 1.f, err = INFINITY;
+    bool running = has_rows;
+    for (int it = 0; it < maxiter; ++it) {
+      if (it > 0) running = running && (err > tol);
+      if (!running) break;
+      // gradient at y: r = A y + b, g = A^T r
+      apply([&](int i, int k) { return Y[i][k]; }, [&](int k) { return yl[k]; },
+            [&](int i, int k, float o) { R[i][k] = o + sb[i][k]; },
+            [&](int k, float o) { rl[k] = o + lb[k]; });
+      apply([&](int i, int k) { return R[i][k]; }, [&](int k) { return rl[k]; },
+            [&](int i, int k, float o) { G[i][k] = o; }, [&](int k, float o) { gl[k] = o; });
+      // line search over x+ = relu(y - eta g).  f is quadratic, so with
+      // d = x+ - y its test f(x+) - f(y) > g.d + |d|^2 / (2 eta) is
+      // |A d|^2 / 2 > |d|^2 / (2 eta): without the difference of two nearly
+      // equal sums, rounding does not decide a step.  R holds A d.
+      bool cond = true;
+      for (int ls = 0; ls <= maxls && cond; ++ls) {
+        if (ls > 0) eta *= 0.5f;
+        const float e_ = eta;
+        float ad = 0.f, dd = 0.f;
+        apply([&](int i, int k) { return fmaxf(Y[i][k] - e_ * G[i][k], 0.f) - Y[i][k]; },
+              [&](int k) { return fmaxf(yl[k] - e_ * gl[k], 0.f) - yl[k]; },
+              [&](int i, int k, float o) {
+                R[i][k] = o;
+                ad += o * o;
+                const float d = fmaxf(Y[i][k] - e_ * G[i][k], 0.f) - Y[i][k];
+                dd += d * d;
+              },
+              [&](int k, float o) {
+                rl[k] = o;
+                ad += o * o;
+                const float d = fmaxf(yl[k] - e_ * gl[k], 0.f) - yl[k];
+                dd += d * d;
+              });
+        ad = quad_sum(ad), dd = quad_sum(dd);
+        trials += 1;
+        cond = e_ * (0.5f * ad) > 0.5f * dd + lseps;
+      }
+      // error at x+: |relu(x+ - grad f(x+)) - x+|, grad f(x+) = g + A^T A d
+      const float e_ = eta;
+      float e2 = 0.f;
+      apply([&](int i, int k) { return R[i][k]; }, [&](int k) { return rl[k]; },
+            [&](int i, int k, float o) {
+              const float xn = fmaxf(Y[i][k] - e_ * G[i][k], 0.f);
+              const float dv = fmaxf(xn - (G[i][k] + o), 0.f) - xn;
+              e2 += dv * dv;
+            },
+            [&](int k, float o) {
+              const float xn = fmaxf(yl[k] - e_ * gl[k], 0.f);
+              const float dv = fmaxf(xn - (gl[k] + o), 0.f) - xn;
+              e2 += dv * dv;
+            });
+      err = fsqrt(quad_sum(e2));
+      const float tn = 0.5f * (1.f + fsqrt(1.f + 4.f * tk * tk));
+      const float beta = (tk - 1.f) * rcp(tn);
+#pragma unroll
+      for (int i = 0; i < S; ++i)
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+          const float xn = fmaxf(Y[i][k] - e_ * G[i][k], 0.f);
+          Y[i][k] = xn + beta * (xn - X[i][k]);
+          X[i][k] = xn;
+        }
+#pragma unroll
+      for (int k = 0; k < K; ++k) {
+        const float xn = fmaxf(yl[k] - e_ * gl[k], 0.f);
+        yl[k] = xn + beta * (xn - xl[k]);
+        xl[k] = xn;
+      }
+      eta = eta <= 1e-6f ? 1.f : eta * 2.f;
+      tk = tn;
+      iters += 1;
+    }
+    // ---- qdd = u + L^-1 (L^-T J^T) x (integrator.py:58-64)
+    float t[K], tr[6];
+    gather([&](int i, int k) { return X[i][k]; }, [&](int k) { return xl[k]; }, t, tr);
+    F.l(t, tr);
+#pragma unroll
+    for (int k = 0; k < K; ++k) u[k] = has_rows ? u[k] + t[k] : u[k];
+#pragma unroll
+    for (int k = 0; k < 6; ++k) ur[k] = has_rows ? ur[k] + tr[k] : ur[k];
+  }
+  if (probe) {
+#pragma unroll
+    for (int k = 0; k < K; ++k) probe[NV + 6 + b * K + k] = u[k];
+    if (b == 0) {
+#pragma unroll
+      for (int k = 0; k < 6; ++k) probe[NV + k] = ur[k];
+      probe[2 * NV] = (float)n_c;
+      probe[2 * NV + 1] = (float)iters;
+      probe[2 * NV + 2] = (float)trials;
+    }
+  }
+
+  // ---- semi-implicit Euler (integrator.py:26-84)
+  const float dt = ml[H_DT];
+#pragma unroll
+  for (int k = 0; k < K; ++k) {
+    s.qd[k] = s.qd[k] + u[k] * dt;
+    s.q[k] = s.q[k] + s.qd[k] * dt;
+  }
+#pragma unroll
+  for (int k = 0; k < 6; ++k) s.rv[k] = s.rv[k] + ur[k] * dt;
+  const Q4 rot = integrate_rot(Q4{s.rq[3], s.rq[4], s.rq[5], s.rq[6]},
+                               v3(s.rv[3], s.rv[4], s.rv[5]), dt);
+  s.rq[3] = rot.w, s.rq[4] = rot.x, s.rq[5] = rot.y, s.rq[6] = rot.z;
+#pragma unroll
+  for (int k = 0; k < 3; ++k) s.rq[k] = s.rq[k] + s.rv[k] * dt;
+  return n_c;
+}
+
+// a pointer known to be LDS again after a call that is not inlined
+BGX_D float* star_lds(float* p) { return (float*)(__attribute__((address_space(3))) float*)p; }
+
+// The frames of an env's state (pipeline.init's x, xd).  A function of its
+// own, so that a step's frames and init's are the same code: bitwise equal.
+template <class T>
+BGX_ITEM void star_write_frames(const Launch& a, long long env, int b, float* lds,
+                                StarState<T> s, bool live) {
+  constexpr int K = Star<T>::K;
+  const float* ml = star_lds(lds);
+  V3 xp0, xp[K], xa0, xa[K], xv[K];
+  Q4 xr0, xr[K];
+  star_frames<T, true>(ml, b, s, xp0, xr0, xp, xr, &xa0, xa, xv);
+  if (!live) return;
+  const long long o = env * T::L, ol = o + 1 + b * K;
+  auto put3 = [&](float* base, V3 root, const V3* leg) {
+    if (!base) return;
+    if (b < 3) base[3 * o + b] = by_leg(b, root.x, root.y, root.z, 0.f);
+#pragma unroll
+    for (int k = 0; k < K; ++k) {
+      float* p = base + 3 * (ol + k);
+      p[0] = leg[k].x, p[1] = leg[k].y, p[2] = leg[k].z;
+    }
+  };
+  put3(a.x_pos, xp0, xp);
+  if (a.x_rot) {
+    a.x_rot[4 * o + b] = by_leg(b, xr0.w, xr0.x, xr0.y, xr0.z);
+#pragma unroll
+    for (int k = 0; k < K; ++k) {
+      float* p = a.x_rot + 4 * (ol + k);
+      p[0] = xr[k].w, p[1] = xr[k].x, p[2] = xr[k].y, p[3] = xr[k].z;
+    }
+  }
+  put3(a.xd_ang, xa0, xa);
+  put3(a.xd_vel, v3(s.rv[0], s.rv[1], s.rv[2]), xv);
+}
+
+// the model table at M into LDS (a wavefront's workgroup)
+template <class T>
+BGX_D void star_stage(const float* M, float* lds) {
+  for (int i = threadIdx.x; i < T::SIZE; i += WAVE) lds[i] = M[i];
+  __syncthreads();
+}
+
+// The envs of one item (up to STAR_ENVS), n_steps x n_frames substeps.  An
+// env past the item's count computes on the item's last env and writes
+// nothing.  A function of its own (as chain_item): the homogeneous kernel and
+// the batch kernel call the same code.
+template <class T>
+BGX_ITEM void star_item(const Launch& a, const BatchItem& it, float* lds_) {
+  constexpr int K = Star<T>::K, NQ = T::NQ, NV = T::NV, NU = T::NU;
+  float* lds = star_lds(lds_);
+  const int b = threadIdx.x % STAR_LEGS, e = threadIdx.x / STAR_LEGS;
+  const bool live = e < it.n;
+  const int ec = live ? e : it.n - 1;
+  const long long env = it.env + ec;
+  star_stage<T>(a.M + it.m_off, lds);
+  float* qp = a.q + it.q + (long long)ec * NQ;
+  float* qdp = a.qd + it.qd + (long long)ec * NV;
+  const float* actp = (NU > 0 && a.act) ? a.act + it.act + (long long)ec * NU : nullptr;
+  const long long n_sub = (long long)a.n_steps * a.n_frames, seg = blockIdx.y;
+  float* subq = (live && a.sub_q) ? a.sub_q + (seg * n_sub * a.n + env) * NQ : nullptr;
+  float* subqd = (live && a.sub_qd) ? a.sub_qd + (seg * n_sub * a.n + env) * NV : nullptr;
+  float* probe = (live && a.probe) ? a.probe + env * (2 * NV + 3) : nullptr;
+  StarState<T> s;
+  star_load(s, b, qp, qdp);
+  const int n_steps = a.n_steps, n_frames = a.n_frames;
+  int st = 0;
+  for (int t = 0; t < n_steps; ++t) {
+    float act[K];
+#pragma unroll
+    for (int k = 0; k < K; ++k) {
+      act[k] = 0.f;
+      if (star_act<T>(6 + k) >= 0) {
+        if (actp) act[k] = actp[t * a.act_stride + star_act_of_leg<T>(b, k)];
+      }
+    }
+    for (int f = 0; f < n_frames; ++f) {
+      if (subq) {
+        const long long o = ((long long)t * n_frames + f) * a.n;
+        star_store_q(s, b, subq + o * NQ);
+        star_store_qd(s, b, subqd + o * NV);
+      }
+      // the status of the one-thread kernel: more contacts than its slots
+      if (star_substep<T>(lds, b, s, act, probe) > T::KC) st |= ST_SLOW_PATH;
+    }
+    if (live && a.q_traj) star_store_q(s, b, a.q_traj + t * a.q_step + it.q + (long long)e * NQ);
+    if (live && a.qd_traj)
+      star_store_qd(s, b, a.qd_traj + t * a.qd_step + it.qd + (long long)e * NV);
+  }
+  bool finite = true;
+#pragma unroll
+  for (int k = 0; k < 7; ++k) finite = finite && isfinite(s.rq[k]);
+#pragma unroll
+  for (int k = 0; k < 6; ++k) finite = finite && isfinite(s.rv[k]);
+#pragma unroll
+  for (int k = 0; k < K; ++k) finite = finite && isfinite(s.q[k]) && isfinite(s.qd[k]);
+  if (quad_ballot(!finite) != 0u) st |= ST_NONFINITE;
+  if (live) {
+    star_store_q(s, b, qp);
+    star_store_qd(s, b, qdp);
+    if (a.status && b == 0) {
+      if (a.n_seg > 1) atomicOr(a.status + env, st);
+      else a.status[env] = a.status_or ? (a.status[env] | st) : st;
+    }
+  }
+  if (a.x_pos || a.x_rot || a.xd_ang || a.xd_vel)
+    star_write_frames<T>(a, env, b, lds, s, live);
+}
+
+// the item of a homogeneous launch's workgroup (checkpoint segment blockIdx.y)
+template <class T>
+BGX_D BatchItem star_home_item(const Launch& a) {
+  BatchItem it{};
+  const long long seg = blockIdx.y, env0 = (long long)blockIdx.x * STAR_ENVS;
+  it.kind = BATCH_TREE;
+  it.n = (int)(a.n - env0 < STAR_ENVS ? a.n - env0 : STAR_ENVS);
+  it.env = env0;
+  it.q = (seg * a.n + env0) * T::NQ, it.qd = (seg * a.n + env0) * T::NV;
+  it.act = seg * a.seg_act_stride + env0 * T::NU;
+  return it;
+}
+
+template <class T>
+__global__ __launch_bounds__(WAVE) void k_star(Launch a) {
+  __shared__ __align__(16) float lds[star_lds_floats<T>()];
+  star_item<T>(a, star_home_item<T>(a), lds);
+}
+
+// the batch kernel (bgx_batch.h) of a topology of this shape
+template <class T>
+__global__ __launch_bounds__(WAVE) void k_star_batch(Launch a) {
+  constexpr int N = star_lds_floats<T>();
+  __shared__ __align__(16) float smem[N > CHAIN_LDS_FLOATS ? N : CHAIN_LDS_FLOATS];
+  for (;;) {
+    const int i = next_item(a);
+    if (i < 0) break;
+    const BatchItem it = a.items[i];
+    if (it.kind == BATCH_CHAIN) run_chain_item(a, it, smem);
+    else star_item<T>(a, it, smem);
+    __syncthreads();  // the next item reuses the LDS
+  }
+  batch_done(a);
+}
+
+template <class T>
+__global__ __launch_bounds__(WAVE) void k_star_init(Launch a) {
+  __shared__ float lds[T::SIZE];
+  const int b = threadIdx.x % STAR_LEGS;
+  const long long env = (long long)blockIdx.x * STAR_ENVS + threadIdx.x / STAR_LEGS;
+  const long long ec = env < a.n ? env : a.n - 1;
+  star_stage<T>(a.M, lds);
+  StarState<T> s;
+  star_load(s, b, a.q + ec * T::NQ, a.qd + ec * T::NV);
+  star_write_frames<T>(a, ec, b, lds, s, env < a.n);
+}
+
+}  // namespace bgx

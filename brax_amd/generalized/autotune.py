@@ -102,8 +102,9 @@ def tune_tile(sys, q: torch.Tensor, qd: torch.Tensor, acts: torch.Tensor, n_fram
   take more LDS per env (fewer workgroups per compute unit); which wins
   depends on the batch's contact counts, which change as the envs settle,
   so acts should span the horizon of interest (a two-step window from
-  standing starts picks too few slots).  Returns the choice, which is set
-  on the model."""
+  standing starts picks too few slots).  Where several lanes per env are the
+  default, that kernel is timed too: choice 0.  Returns the choice, which is
+  set on the model."""
   m = pipeline.device_model(sys, q.device)
   n = q.shape[0]
   key = _key(m, TILE, n, n_frames)
@@ -111,6 +112,8 @@ def tune_tile(sys, q: torch.Tensor, qd: torch.Tensor, acts: torch.Tensor, n_fram
     set_launch(m, TILE, _CACHE[key])
     return _CACHE[key]
   cands = tiles(sys, q.device)
+  if get_launch(m, LANES) > 1:
+    cands = (0,) + cands  # the multi-lane kernel, which has no tile
   if len(cands) == 1:
     set_launch(m, TILE, cands[0])
     _CACHE[key] = cands[0]

@@ -95,9 +95,11 @@ int bgx_model_topology(const bgx_model* model);
 #define BGX_KERNELS_TILE 2
 /* kernels = BGX_KERNELS_LANES sets the step kernels' lanes per env: 1 runs
  * one thread per env; the topology's multi-lane width (the default, 0,
- * where the topology is compiled with the multi-lane tree kernel) runs an
- * env on a group of lanes (a lane per dof).  The two agree within rounding;
- * the getter returns the width in use. */
+ * where the topology is compiled with a multi-lane kernel) runs an env on a
+ * group of lanes: 4 for a free root with four equal legs (a lane per leg),
+ * a lane per dof for other large trees.  The two agree within rounding; the
+ * getter returns the width.  Choosing an LDS tile runs a four-legged
+ * topology at one thread per env. */
 #define BGX_KERNELS_LANES 3
 /* kernels = BGX_KERNELS_ADJOINT_PARTS splits bgx_rollout_adjoint's backward
  * pass into that many parts of whole envs (1-4; 0 = one), each on its own
