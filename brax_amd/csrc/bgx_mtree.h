@@ -14,9 +14,9 @@
 //    level the other way, children added in the order the serial pass adds
 //    them;
 //  * the mass matrix is built a row per lane (CRBA, mass.py:27-83) and
-//    inverted in place by Gauss-Jordan elimination, one pivot per step with
-//    the pivot row broadcast through LDS, so that M^-1 v is one broadcast
-//    matrix-vector product with no serial chain;
+//    inverted in registers by Gauss-Jordan elimination, one pivot per step
+//    with the pivot row broadcast through LDS, so that M^-1 v is one
+//    broadcast matrix-vector product with no serial chain;
 //  * a candidate's four contact rows and a dof's limit row sit on their
 //    lanes (an inactive candidate's rows are zero, which leaves every
 //    projected-gradient iterate as if they were dropped, constraint.py:174),
@@ -114,25 +114,22 @@ struct MTab {
     for (int c = 0; c < NC; ++c) m = tab.npath[c] > m ? tab.npath[c] : m;
     return m;
   }();
-  // LDS of one env (floats)
-  static constexpr int LJ = 0;            // [L][7] joint transforms (pos, rot)
-  static constexpr int LX = LJ + 7 * L;   // [L][7] world frames
-  static constexpr int CDF = LX + 7 * L;  // [NV][6] cdof (ang, vel)
-  static constexpr int ZV = CDF + 6 * NV;  // [NV] a per-dof vector
-  static constexpr int LA = ZV + NV;      // [L][6] link velocities / accelerations
-  static constexpr int LB = LA + 6 * L;   // [L][6] link velocities at qd
-  static constexpr int LF = LB + 6 * L;   // [L][6] subtree sums
-  static constexpr int CF = LF + 6 * L;   // [NC][6] candidate forces (torque, force)
-  static constexpr int PV = CF + 6 * (NC > 0 ? NC : 1);  // [2][NV] pivot rows
-  static constexpr int CI = PV + 2 * NV;  // [L][10] composite inertias (cc, ci, mass)
-  static constexpr int FS = CI + 10 * L;  // [NV][6] I_c cdof
-  static constexpr int QS = FS + 6 * NV;  // [NQ + NV] the state, for the frames
-  static constexpr int ZW = QS + NQ + NV;  // [NV] a second per-dof vector
-  // M, then M^-1, row d at MI + d MIS (an odd stride: lanes reading their
-  // rows hit distinct banks)
-  static constexpr int MIS = NV % 2 ? NV + 2 : NV + 1;
-  static constexpr int MI = ZW + NV;
-  static constexpr int SIZE = MI + NV * MIS;
+  // LDS of one env (floats).  Vectors that every lane reads are padded to
+  // float4s: a row of NVP, an (angular, linear) pair of 8
+  static constexpr int NVP = (NV + 3) / 4 * 4;
+  static constexpr int PV = 0;               // [2][NVP] pivot rows
+  static constexpr int ZV = PV + 2 * NVP;    // [NVP] a per-dof vector
+  static constexpr int ZW = ZV + NVP;        // [NVP] a second per-dof vector
+  static constexpr int CDF = ZW + NVP;       // [NV][8] cdof (ang, vel)
+  static constexpr int FS = CDF + 8 * NV;    // [NV][8] I_c cdof
+  static constexpr int CF = FS + 8 * NV;     // [NC][8] candidate forces (torque, force)
+  static constexpr int LX = CF + 8 * (NC > 0 ? NC : 1);  // [L][7] world frames
+  static constexpr int LA = LX + 7 * L;      // [L][6] link velocities / accelerations
+  static constexpr int LB = LA + 6 * L;      // [L][6] link velocities at qd
+  static constexpr int LF = LB + 6 * L;      // [L][6] subtree sums
+  static constexpr int CI = LF + 6 * L;      // [L][10] composite inertias (cc, ci, mass)
+  static constexpr int QS = CI + 10 * L;     // [NQ + NV] the state, for the frames
+  static constexpr int SIZE = (QS + NQ + NV + 3) / 4 * 4;
 };
 
 // whether topology T can run the multi-lane tree kernel
@@ -162,6 +159,25 @@ BGX_D bool wave_any(bool b) { return __ballot(b) != 0ull; }
 
 BGX_D V3 ld3l(const float* p) { return v3(p[0], p[1], p[2]); }
 BGX_D Q4 ld4l(const float* p) { return Q4{p[0], p[1], p[2], p[3]}; }
+// x where bit k of m is set, else 0 (no compare: 36 lane masks kept over the
+// solver's loops would spill)
+BGX_D float masked(float x, unsigned m, int k) {
+  return __builtin_bit_cast(float, __builtin_bit_cast(int, x) & ((int)(m << (31 - k)) >> 31));
+}
+// 16-byte aligned LDS: a pair's half, and row j / 4 of a padded vector
+BGX_D V3 ld3a(const float* p) {
+  const float4 f = *(const float4*)p;
+  return v3(f.x, f.y, f.z);
+}
+BGX_D void st3a(float* p, V3 v) { *(float4*)p = float4{v.x, v.y, v.z, 0.f}; }
+template <int N>
+BGX_D void ldrow(const float* p, float* v) {
+#pragma unroll
+  for (int j = 0; j < N; j += 4) {
+    const float4 f = *(const float4*)(p + j);
+    v[j] = f.x, v[j + 1] = f.y, v[j + 2] = f.z, v[j + 3] = f.w;
+  }
+}
 BGX_D void st3l(float* p, V3 v) { p[0] = v.x, p[1] = v.y, p[2] = v.z; }
 BGX_D void st4l(float* p, Q4 v) { p[0] = v.w, p[1] = v.x, p[2] = v.y, p[3] = v.z; }
 
@@ -347,9 +363,9 @@ BGX_D void mtree_substep(const float* __restrict__ M, MLane<T>& s, const float* 
     aa = rotate(aa, jr);
     ca = aa;
     cv = vv - cross(rc - jp, aa);
-    float* cf = lds + MT::CDF + 6 * d;
-    st3l(cf, ca);
-    st3l(cf + 3, cv);
+    float* cf = lds + MT::CDF + 8 * d;
+    st3a(cf, ca);
+    st3a(cf + 4, cv);
   }
   __syncthreads();  // the hinge coordinates in ZV are read; qd replaces them
   if (d >= 0) lds[MT::ZV + d] = s.qd;
@@ -372,10 +388,10 @@ BGX_D void mtree_substep(const float* __restrict__ M, MLane<T>& s, const float* 
         for (int k = 0; k < 6; ++k) {
           if (k < nd) {
             const int dd = T::DADR[ll] + k;
-            const float* cf = lds + MT::CDF + 6 * dd;
+            const float* cf = lds + MT::CDF + 8 * dd;
             const float z = lds[MT::ZV + dd];
-            a = a + ld3l(cf) * z;
-            v = v + ld3l(cf + 3) * z;
+            a = a + ld3a(cf) * z;
+            v = v + ld3a(cf + 4) * z;
           }
         }
         va = a, vv = v;
@@ -433,8 +449,8 @@ BGX_D void mtree_substep(const float* __restrict__ M, MLane<T>& s, const float* 
         a = ld3l(pf), v = ld3l(pf + 3);
       }
       auto cdof_of = [&](int dd, V3& oa, V3& ov) {
-        const float* cf = lds + MT::CDF + 6 * dd;
-        oa = ld3l(cf), ov = ld3l(cf + 3);
+        const float* cf = lds + MT::CDF + 8 * dd;
+        oa = ld3a(cf), ov = ld3a(cf + 4);
       };
       auto qd_of = [&](int dd) { return lds[MT::ZV + dd]; };
       if (T::LTYPE[ll] == 0) {
@@ -543,53 +559,61 @@ BGX_D void mtree_substep(const float* __restrict__ M, MLane<T>& s, const float* 
     const float* cf = lds + MT::CI + 10 * dlc;
     inertia_mul(ld3l(cf), Sym3{cf[3], cf[4], cf[5], cf[6], cf[7], cf[8]}, cf[9], ca, cv, Fa,
                 Fv);
-    float* fs = lds + MT::FS + 6 * d;
-    st3l(fs, Fa);
-    st3l(fs + 3, Fv);
+    float* fs = lds + MT::FS + 8 * d;
+    st3a(fs, Fa);
+    st3a(fs + 4, Fv);
   }
   __syncthreads();
-  float* mrow = lds + MT::MI + (d >= 0 ? d : 0) * MT::MIS;  // row d of M, then of M^-1
+  float mrow[MT::NVP];  // row d of M, then of M^-1
+#pragma unroll
+  for (int j = NV; j < MT::NVP; ++j) mrow[j] = 0.f;
   {
     const unsigned danc = d >= 0 ? T::DANC[d] : 0u;
     const float arm = d >= 0 ? dof_rec<T>(M, d)[DF_ARMATURE] : 1.f;
-#pragma unroll 2
+#pragma unroll
     for (int j = 0; j < NV; ++j) {
-      const float* cf = lds + MT::CDF + 6 * j;
-      const float* fs = lds + MT::FS + 6 * j;
-      const float lower = dot(ld3l(cf + 3), Fv) + dot(ld3l(cf), Fa);
-      const float upper = dot(cv, ld3l(fs + 3)) + dot(ca, ld3l(fs));
+      const float* cf = lds + MT::CDF + 8 * j;
+      const float* fs = lds + MT::FS + 8 * j;
+      const float lower = dot(ld3a(cf + 4), Fv) + dot(ld3a(cf), Fa);
+      const float upper = dot(cv, ld3a(fs + 4)) + dot(ca, ld3a(fs));
       const bool in_lower = j < d && ((danc >> j) & 1u);
       const bool in_upper = j > d && ((T::DANC[j] >> (d >= 0 ? d : 0)) & 1u);
-      const float mj = j == d ? (dot(cv, Fv) + dot(ca, Fa)) + arm
-                              : (in_lower ? lower : (in_upper ? upper : 0.f));
-      if (d >= 0) mrow[j] = mj;
+      mrow[j] = j == d ? (dot(cv, Fv) + dot(ca, Fa)) + arm
+                       : (in_lower ? lower : (in_upper ? upper : 0.f));
+      // four columns' reads in flight, not all of them
+      if (j % 4 == 3) asm volatile("" ::: "memory");
     }
   }
   // ---- M^-1 in place by Gauss-Jordan elimination (M is positive definite:
-  // no pivoting), row d on lane d, the pivot row read by every lane
-#pragma unroll 1
+  // no pivoting), row d on lane d in registers; the pivot row goes through
+  // LDS, two buffers in turn so that one barrier a pivot is enough.  Rows in
+  // LDS cost three LDS accesses per entry and pivot, 1,600 of a substep's
+  // accesses, on a kernel that LDS issue bounds.
+#pragma unroll
   for (int k = 0; k < NV; ++k) {
-    __syncthreads();
-    const float* prow = lds + MT::MI + k * MT::MIS;
-    const float pk = rcp(prow[k]);
-    __syncthreads();  // every lane has the pivot before row k changes
+    float* pb = lds + MT::PV + (k & 1) * MT::NVP;
     if (d == k) {
-#pragma unroll 4
-      for (int j = 0; j < NV; ++j) mrow[j] = j == k ? pk : mrow[j] * pk;
+#pragma unroll
+      for (int j = 0; j < MT::NVP; j += 4)
+        *(float4*)(pb + j) = float4{mrow[j], mrow[j + 1], mrow[j + 2], mrow[j + 3]};
     }
     __syncthreads();
-    if (d >= 0 && d != k) {
-      const float f = mrow[k];
-#pragma unroll 4
-      for (int j = 0; j < NV; ++j) mrow[j] = j == k ? -f * pk : mrow[j] - f * prow[j];
-    }
+    float prow[MT::NVP];
+    ldrow<MT::NVP>(pb, prow);
+    const float pk = rcp(prow[k]);
+    const bool own = d == k;
+    const float f = own ? -1.f : mrow[k];
+#pragma unroll
+    for (int j = 0; j < NV; ++j)
+      mrow[j] = j == k ? (own ? pk : -f * pk) : (own ? 0.f : mrow[j]) - f * (prow[j] * pk);
   }
-  __syncthreads();
   // M^-1 times the per-dof vector in ZV, on this dof
   auto minv_mul = [&]() {
+    float v[MT::NVP];
+    ldrow<MT::NVP>(lds + MT::ZV, v);
     float z = 0.f;
 #pragma unroll
-    for (int j = 0; j < NV; ++j) z += mrow[j] * lds[MT::ZV + j];
+    for (int j = 0; j < NV; ++j) z += mrow[j] * v[j];
     return z;
   };
   // the velocity (angular, linear) of candidate c's link under the per-dof
@@ -597,14 +621,12 @@ BGX_D void mtree_substep(const float* __restrict__ M, MLane<T>& s, const float* 
   // order of dynamics.py:93-103's scan)
   auto path_vel = [&](int base, V3& wa, V3& wv) {
     wa = v3zero(), wv = v3zero();
-#pragma unroll
+#pragma unroll 4
     for (int dd = 0; dd < NV; ++dd) {  // ancestors first: dof indices grow down the tree
-      if ((s.pmask >> dd) & 1u) {
-        const float* cf = lds + MT::CDF + 6 * dd;
-        const float z = lds[base + dd];
-        wa = wa + ld3l(cf) * z;
-        wv = wv + ld3l(cf + 3) * z;
-      }
+      const float* cf = lds + MT::CDF + 8 * dd;
+      const float z = masked(lds[base + dd], s.pmask, dd);  // no branch: the reads pipeline
+      wa = wa + ld3a(cf) * z;
+      wv = wv + ld3a(cf + 4) * z;
     }
   };
   // ---- u = M^-1 qf_smooth
@@ -688,21 +710,20 @@ BGX_D void mtree_substep(const float* __restrict__ M, MLane<T>& s, const float* 
       const V3 w = d0 * ((in[0] + in[1]) + (in[2] + in[3])) + d1 * (in[0] - in[1]) +
                    d2 * (in[2] - in[3]);
       const V3 ta = cross(r, w);
-      float* cf = lds + MT::CF + 6 * cc_;
-      st3l(cf, active ? ta : v3zero());
-      st3l(cf + 3, active ? w : v3zero());
+      float* cf = lds + MT::CF + 8 * cc_;
+      st3a(cf, active ? ta : v3zero());
+      st3a(cf + 4, active ? w : v3zero());
     }
     __syncthreads();
     // the dof's generalized force: its cdof against the forces of the
     // candidates on its subtree (dynamics.py:174-182's sums, gathered)
     float tau = 0.f;
     if (d >= 0) {
-#pragma unroll
+#pragma unroll 4
       for (int k = 0; k < NC; ++k) {
-        if ((s.cmask >> k) & 1u) {
-          const float* cf = lds + MT::CF + 6 * k;
-          tau += dot(cv, ld3l(cf + 3)) + dot(ca, ld3l(cf));
-        }
+        const float* cf = lds + MT::CF + 8 * k;
+        const float f = dot(cv, ld3a(cf + 4)) + dot(ca, ld3a(cf));
+        tau += masked(f, s.cmask, k);
       }
       tau += lside * in_l;
       lds[MT::ZV + d] = tau;
@@ -751,11 +772,6 @@ BGX_D void mtree_substep(const float* __restrict__ M, MLane<T>& s, const float* 
         if (running) Rr[k] = active ? o[k] + sb[k] : 0.f;
       if (running) rl = ol + lb;
     }
-    float fy = 0.f;
-#pragma unroll
-    for (int k = 0; k < 4; ++k) fy += active ? 0.5f * Rr[k] * Rr[k] : 0.f;
-    fy += has_l ? 0.5f * rl * rl : 0.f;
-    fy = gsum<G>(fy);
     {
       apply_a(Rr, rl, o, ol);
 #pragma unroll
@@ -763,7 +779,10 @@ BGX_D void mtree_substep(const float* __restrict__ M, MLane<T>& s, const float* 
         if (running) Gr[k] = o[k];
       if (running) gl = ol;
     }
-    // line search: trial x+ = relu(y - eta g), residual into r
+    // line search over x+ = relu(y - eta g), the test in terms of A d,
+    // d = x+ - y (bgx_star.h): f(x+) - f(y) > g.d + |d|^2 / (2 eta) is
+    // |A d|^2 / 2 > |d|^2 / (2 eta), where rounding decides no step.  R
+    // becomes A d.
     bool cond = running;
     for (int ls = 0; ls <= maxls; ++ls) {
       if (!wave_any(cond)) break;
@@ -771,34 +790,26 @@ BGX_D void mtree_substep(const float* __restrict__ M, MLane<T>& s, const float* 
       const float e_ = eta;
       float in[4], in_l;
 #pragma unroll
-      for (int k = 0; k < 4; ++k) in[k] = fmaxf(Y[k] - e_ * Gr[k], 0.f);
-      in_l = fmaxf(yl - e_ * gl, 0.f);
+      for (int k = 0; k < 4; ++k) in[k] = fmaxf(Y[k] - e_ * Gr[k], 0.f) - Y[k];
+      in_l = fmaxf(yl - e_ * gl, 0.f) - yl;
       apply_a(in, in_l, o, ol);
-      float fx = 0.f, dg = 0.f, dd = 0.f;
+      float ad = 0.f, dd = 0.f;
 #pragma unroll
       for (int k = 0; k < 4; ++k) {
-        const float rv = o[k] + sb[k];
-        if (cond) Rr[k] = rv;
-        const float df = in[k] - Y[k];
-        fx += active ? 0.5f * rv * rv : 0.f;
-        dg += active ? df * Gr[k] : 0.f;
-        dd += active ? df * df : 0.f;
+        if (cond) Rr[k] = o[k];
+        ad += active ? o[k] * o[k] : 0.f;
+        dd += active ? in[k] * in[k] : 0.f;
       }
-      {
-        const float rv = ol + lb;
-        if (cond) rl = rv;
-        const float df = in_l - yl;
-        fx += has_l ? 0.5f * rv * rv : 0.f;
-        dg += has_l ? df * gl : 0.f;
-        dd += has_l ? df * df : 0.f;
-      }
-      fx = gsum<G>(fx), dg = gsum<G>(dg), dd = gsum<G>(dd);
+      if (cond) rl = ol;
+      ad += has_l ? ol * ol : 0.f;
+      dd += has_l ? in_l * in_l : 0.f;
+      ad = gsum<G>(ad), dd = gsum<G>(dd);
       if (cond) {
         trials += 1;
-        cond = e_ * (fx - fy) > e_ * dg + 0.5f * dd + lseps;
+        cond = e_ * (0.5f * ad) > 0.5f * dd + lseps;
       }
     }
-    // error at x+: |relu(x+ - grad f(x+)) - x+| with grad = A^T (A x+ + b)
+    // error at x+: |relu(x+ - grad f(x+)) - x+|, grad f(x+) = g + A^T A d
     const float e_ = eta;
     apply_a(Rr, rl, o, ol);
     float e2 = 0.f;
@@ -806,12 +817,12 @@ BGX_D void mtree_substep(const float* __restrict__ M, MLane<T>& s, const float* 
 #pragma unroll
     for (int k = 0; k < 4; ++k) {
       xp[k] = fmaxf(Y[k] - e_ * Gr[k], 0.f);
-      const float dv = fmaxf(xp[k] - o[k], 0.f) - xp[k];
+      const float dv = fmaxf(xp[k] - (Gr[k] + o[k]), 0.f) - xp[k];
       e2 += active ? dv * dv : 0.f;
     }
     xpl = fmaxf(yl - e_ * gl, 0.f);
     {
-      const float dv = fmaxf(xpl - ol, 0.f) - xpl;
+      const float dv = fmaxf(xpl - (gl + ol), 0.f) - xpl;
       e2 += has_l ? dv * dv : 0.f;
     }
     e2 = gsum<G>(e2);
@@ -824,13 +835,10 @@ BGX_D void mtree_substep(const float* __restrict__ M, MLane<T>& s, const float* 
         const float xk = active ? xp[k] : 0.f;
         Y[k] = active ? xk + beta * (xk - X[k]) : 0.f;
         X[k] = xk;
-        // the next y's gradient; o holds A (A x+ + b)
-
       }
       if (has_l) {
         yl = xpl + beta * (xpl - xl);
         xl = xpl;
-
       }
       eta = eta <= 1e-6f ? 1.f : eta * 2.f;
       tk = tn;
@@ -893,7 +901,7 @@ template <class T>
 __global__ __launch_bounds__(WAVE) __attribute__((amdgpu_waves_per_eu(3))) void k_mtree(Launch a) {
   using MT = MTab<T>;
   constexpr int G = MT::G, E = MT::E, NQ = T::NQ, NV = T::NV, NU = T::NU;
-  __shared__ float smem[E * MT::SIZE];
+  __shared__ __align__(16) float smem[E * MT::SIZE];
   const int wl = threadIdx.x, g = wl % G, gb = wl - g, e = wl / G;
   const long long env = (long long)blockIdx.x * E + e;
   const bool live = env < a.n;
