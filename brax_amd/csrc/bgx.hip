@@ -228,6 +228,33 @@ int bgx_init(const bgx_model* m, int32_t n, const float* q, const float* qd, flo
   return launch(m, true, a, stream);
 }
 
+int bgx_init_copy(const bgx_model* m, int32_t n, const float* q_in, const float* qd_in, float* q,
+                  float* qd, float* x_pos, float* x_rot, float* xd_ang, float* xd_vel,
+                  void* stream) {
+  if (n > 0 && (!q_in || !qd_in)) return fail(BGX_ERR_ARG, "q/qd must be non-null");
+  bgx::Launch a{};
+  a.n = n;
+  a.q = q, a.qd = qd, a.q_in = q_in, a.qd_in = qd_in;
+  a.x_pos = x_pos, a.x_rot = x_rot, a.xd_ang = xd_ang, a.xd_vel = xd_vel;
+  return launch(m, true, a, stream);
+}
+
+int bgx_rollout_from(const bgx_model* m, int32_t n, int32_t n_steps, int32_t n_frames,
+                     const float* q_in, const float* qd_in, float* q, float* qd,
+                     const float* act, int64_t act_step_stride, float* q_traj, float* qd_traj,
+                     float* x_pos, float* x_rot, float* xd_ang, float* xd_vel, int32_t* status,
+                     void* stream) {
+  if (n > 0 && (!q_in || !qd_in)) return fail(BGX_ERR_ARG, "q/qd must be non-null");
+  bgx::Launch a{};
+  a.n = n, a.n_steps = n_steps, a.n_frames = n_frames;
+  a.q = q, a.qd = qd, a.q_in = q_in, a.qd_in = qd_in;
+  a.act = act, a.act_stride = act_step_stride;
+  a.q_traj = q_traj, a.qd_traj = qd_traj;
+  a.x_pos = x_pos, a.x_rot = x_rot, a.xd_ang = xd_ang, a.xd_vel = xd_vel;
+  a.status = status;
+  return launch(m, false, a, stream);
+}
+
 int bgx_step(const bgx_model* m, int32_t n, int32_t n_frames, float* q, float* qd,
              const float* act, float* x_pos, float* x_rot, float* xd_ang, float* xd_vel,
              int32_t* status, void* stream) {

@@ -65,8 +65,8 @@ BGX_ITEM void chain_item(const Launch& a, const BatchItem& b, float* lds) {
   const bool dof = l < L;
   float* qp = a.q + b.q + (long long)ec * L;
   float* qdp = a.qd + b.qd + (long long)ec * L;
-  float q = dof ? qp[l] : 0.f;
-  float qd = dof ? qdp[l] : 0.f;
+  float q = dof ? (a.q_in ? a.q_in[b.q + (long long)ec * L + l] : qp[l]) : 0.f;
+  float qd = dof ? (a.qd_in ? a.qd_in[b.qd + (long long)ec * L + l] : qdp[l]) : 0.f;
   float* probe = (live && a.probe) ? a.probe + (b.env + e) * (2 * L + 3) : nullptr;
   for (int s = 0; s < a.n_steps; ++s) {
     const float* ar = a.act ? a.act + s * a.act_stride + b.act + (long long)ec * L : nullptr;

@@ -22,8 +22,10 @@ __global__ __launch_bounds__(WAVE) void k_chain_init(Launch a, int L) {
   const float* M = a.M + ec * chain_table_size(L);
   const ChainLink c = chain_link(M, L, l);
   const bool dof = l < L;
-  const float q = dof ? a.q[ec * L + l] : 0.f;
-  const float qd = dof ? a.qd[ec * L + l] : 0.f;
+  const float q = dof ? (a.q_in ? a.q_in : a.q)[ec * L + l] : 0.f;
+  const float qd = dof ? (a.qd_in ? a.qd_in : a.qd)[ec * L + l] : 0.f;
+  if (live && dof && a.q_in) a.q[env * L + l] = q;
+  if (live && dof && a.qd_in) a.qd[env * L + l] = qd;
   V3 xp, xa, xv;
   Q4 xr;
   chain_frames_xd<G>(l, c, q, qd, xp, xr, xa, xv);
@@ -70,8 +72,11 @@ hipError_t chain_rollout(const Launch& a, hipStream_t s) {
                      dim3((unsigned)(per * G)), 0, s, h);
   hipError_t e = hipGetLastError();
   if (e != hipSuccess) return e;
-  // frames at the new state (the rollout updated q, qd in place)
-  if (a.x_pos || a.x_rot || a.xd_ang || a.xd_vel) return chain_init<L>(a, s);
+  // frames at the new state (the rollout left it in q, qd)
+  if (a.x_pos || a.x_rot || a.xd_ang || a.xd_vel) {
+    h.q_in = h.qd_in = nullptr;
+    return chain_init<L>(h, s);
+  }
   return hipSuccess;
 }
 

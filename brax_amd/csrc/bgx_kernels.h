@@ -88,9 +88,17 @@ __global__ __launch_bounds__(WAVE) void k_init(Launch a) {
   if (env >= a.n) return;
   float q[T::NQ], qd[T::NV];
 #pragma unroll
-  for (int k = 0; k < T::NQ; ++k) q[k] = a.q[(long long)env * T::NQ + k];
+  for (int k = 0; k < T::NQ; ++k) q[k] = (a.q_in ? a.q_in : a.q)[(long long)env * T::NQ + k];
 #pragma unroll
-  for (int k = 0; k < T::NV; ++k) qd[k] = a.qd[(long long)env * T::NV + k];
+  for (int k = 0; k < T::NV; ++k) qd[k] = (a.qd_in ? a.qd_in : a.qd)[(long long)env * T::NV + k];
+  if (a.q_in) {
+#pragma unroll
+    for (int k = 0; k < T::NQ; ++k) a.q[(long long)env * T::NQ + k] = q[k];
+  }
+  if (a.qd_in) {
+#pragma unroll
+    for (int k = 0; k < T::NV; ++k) a.qd[(long long)env * T::NV + k] = qd[k];
+  }
   write_frames<T>(a, env, q, qd);
 }
 
@@ -156,9 +164,9 @@ BGX_D void tree_item(const Launch& a, const BatchItem& b, float* smem) {
   float* lds = smem + threadIdx.x;
   float q[NQ], qd[NV];
 #pragma unroll
-  for (int k = 0; k < NQ; ++k) q[k] = qp[k];
+  for (int k = 0; k < NQ; ++k) q[k] = a.q_in ? a.q_in[b.q + (long long)i * NQ + k] : qp[k];
 #pragma unroll
-  for (int k = 0; k < NV; ++k) qd[k] = qdp[k];
+  for (int k = 0; k < NV; ++k) qd[k] = a.qd_in ? a.qd_in[b.qd + (long long)i * NV + k] : qdp[k];
   float* probe = a.probe ? a.probe + env * (2 * NV + 3) : nullptr;
   int st = 0;
   for (int s = 0; s < a.n_steps; ++s) {
@@ -534,7 +542,9 @@ struct Ops {
                            dim3(WAVE), 0, s, a);
         const hipError_t e = hipGetLastError();
         if (e != hipSuccess || !(a.x_pos || a.x_rot || a.xd_ang || a.xd_vel)) return e;
-        return init(a, s);  // frames of the final state
+        Launch f = a;
+        f.q_in = f.qd_in = nullptr;
+        return init(f, s);  // frames of the final state
       }
     }
     if constexpr (star_ok<T>()) {

@@ -32,6 +32,11 @@ struct Launch {
   int n_frames;
   float* q;
   float* qd;
+  // the initial state, if it is not q and qd themselves: the kernels read it
+  // here and write q and qd (init: copies of it), so that a caller that keeps
+  // its state needs no copy before the launch
+  const float* q_in;
+  const float* qd_in;
   const float* act;
   long long act_stride;
   float* q_traj;   // step s row of an env at q_traj + s * q_step + (its q offset)

@@ -910,8 +910,8 @@ __global__ __launch_bounds__(WAVE) __attribute__((amdgpu_waves_per_eu(3))) void 
   float* lds = smem + e * MT::SIZE;
   const float* M = a.M;
   MLane<T> s = mlane_roles<T>(g, gb);
-  const float* qp = a.q + (seg * a.n + ec) * NQ;
-  const float* qdp = a.qd + (seg * a.n + ec) * NV;
+  const float* qp = (a.q_in ? a.q_in : a.q) + (seg * a.n + ec) * NQ;
+  const float* qdp = (a.qd_in ? a.qd_in : a.qd) + (seg * a.n + ec) * NV;
 #pragma unroll
   for (int k = 0; k < 7; ++k) s.rq[k] = T::LTYPE[0] == 0 ? qp[k] : 0.f;
   s.qh = (s.d >= 0 && T::LTYPE[s.dl] != 0) ? qp[T::QADR[s.dl] + s.dk] : 0.f;

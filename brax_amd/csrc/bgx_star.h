@@ -972,7 +972,8 @@ BGX_ITEM void star_item(const Launch& a, const BatchItem& it, float* lds_) {
   float* subqd = (live && a.sub_qd) ? a.sub_qd + (seg * n_sub * a.n + env) * NV : nullptr;
   float* probe = (live && a.probe) ? a.probe + env * (2 * NV + 3) : nullptr;
   StarState<T> s;
-  star_load(s, b, qp, qdp);
+  star_load(s, b, a.q_in ? a.q_in + it.q + (long long)ec * NQ : qp,
+            a.qd_in ? a.qd_in + it.qd + (long long)ec * NV : qdp);
   const int n_steps = a.n_steps, n_frames = a.n_frames;
   int st = 0;
   for (int t = 0; t < n_steps; ++t) {
@@ -1060,7 +1061,11 @@ __global__ __launch_bounds__(WAVE) void k_star_init(Launch a) {
   const long long ec = env < a.n ? env : a.n - 1;
   star_stage<T>(a.M, lds);
   StarState<T> s;
-  star_load(s, b, a.q + ec * T::NQ, a.qd + ec * T::NV);
+  star_load(s, b, (a.q_in ? a.q_in : a.q) + ec * T::NQ, (a.qd_in ? a.qd_in : a.qd) + ec * T::NV);
+  if (env < a.n) {
+    if (a.q_in) star_store_q(s, b, a.q + env * T::NQ);
+    if (a.qd_in) star_store_qd(s, b, a.qd + env * T::NV);
+  }
   star_write_frames<T>(a, ec, b, lds, s, env < a.n);
 }
 

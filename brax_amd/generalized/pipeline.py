@@ -132,6 +132,12 @@ def _stream():
   return ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)
 
 
+def _state_io(q, qd):
+  """(q, qd) as the kernels read them, and new arrays for the state after."""
+  q_in, qd_in = q.detach().contiguous(), qd.detach().contiguous()
+  return q_in, qd_in, torch.empty_like(q_in), torch.empty_like(qd_in)
+
+
 def _frames(m: DeviceModel, n: int, device):
   return (torch.empty(n, m.L, 3, device=device),
           torch.empty(n, m.L, 4, device=device),
@@ -230,13 +236,15 @@ def init(sys: S.System, q, qd, unused_act=None, unused_ctrl=None,
     qdb = _as_batch(qd, m.nv, m.device, "qd")
     x, xd = frames(sys, qb, qdb)
     return _with_contacts(sys, State(q=qb, qd=qdb, x=x, xd=xd), debug)
-  qb = _as_batch(q, m.nq, m.device, "q").clone()
-  qdb = _as_batch(qd, m.nv, m.device, "qd").clone()
+  q_in = _as_batch(q, m.nq, m.device, "q").detach()
+  qd_in = _as_batch(qd, m.nv, m.device, "qd").detach()
+  qb, qdb = torch.empty_like(q_in), torch.empty_like(qd_in)
   n = qb.shape[0]
   xp, xr, xa, xv = _frames(m, n, m.device)
   lib = _lib.load()
-  _lib.check(lib.bgx_init(m.handle, n, _lib.ptr(qb), _lib.ptr(qdb), _lib.ptr(xp),
-                          _lib.ptr(xr), _lib.ptr(xa), _lib.ptr(xv), _stream()))
+  _lib.check(lib.bgx_init_copy(m.handle, n, _lib.ptr(q_in), _lib.ptr(qd_in), _lib.ptr(qb),
+                               _lib.ptr(qdb), _lib.ptr(xp), _lib.ptr(xr), _lib.ptr(xa),
+                               _lib.ptr(xv), _stream()))
   return _with_contacts(sys, State(q=qb, qd=qdb, x=Transform(xp, xr), xd=Motion(xa, xv)),
                         debug)
 
@@ -280,16 +288,16 @@ def pipeline_step(sys: S.System, state: State, act, n_frames: int = 1,
     q, qd = qt[0], qdt[0]
     x, xd = frames(sys, q, qd)
     return _with_contacts(sys, State(q=q, qd=qd, x=x, xd=xd, status=status), debug)
-  q = state.q.contiguous().clone()
-  qd = state.qd.contiguous().clone()
+  q_in, qd_in, q, qd = _state_io(state.q, state.qd)
   n = q.shape[0]
   a = _act(m, act, n)
   xp, xr, xa, xv = _frames(m, n, m.device)
-  status = torch.zeros(n, dtype=torch.int32, device=m.device)
+  status = torch.empty(n, dtype=torch.int32, device=m.device)
   lib = _lib.load()
-  _lib.check(lib.bgx_step(m.handle, n, int(n_frames), _lib.ptr(q), _lib.ptr(qd),
-                          _lib.ptr(a), _lib.ptr(xp), _lib.ptr(xr), _lib.ptr(xa),
-                          _lib.ptr(xv), _lib.ptr(status), _stream()))
+  _lib.check(lib.bgx_rollout_from(m.handle, n, 1, int(n_frames), _lib.ptr(q_in),
+                                  _lib.ptr(qd_in), _lib.ptr(q), _lib.ptr(qd), _lib.ptr(a), 0,
+                                  None, None, _lib.ptr(xp), _lib.ptr(xr), _lib.ptr(xa),
+                                  _lib.ptr(xv), _lib.ptr(status), _stream()))
   return _with_contacts(sys, State(q=q, qd=qd, x=Transform(xp, xr), xd=Motion(xa, xv),
                                    status=status), debug)
 
@@ -309,8 +317,12 @@ def rollout(sys: S.System, state: State, acts, n_frames: int,
   shape (T, N, q_size) and (T, N, qd_size).
   """
   m = device_model(sys, state.q.device)
-  q = state.q.contiguous().clone()
-  qd = state.qd.contiguous().clone()
+  q_in, qd_in, q, qd = _state_io(state.q, state.qd)
+  if stream is not None:
+    # another stream's launch reads only what the returned State keeps alive
+    q.copy_(q_in)
+    qd.copy_(qd_in)
+    q_in, qd_in = q, qd
   n = q.shape[0]
   acts = torch.as_tensor(acts, dtype=torch.float32, device=m.device)
   if acts.dim() != 3 or acts.shape[1] != n or acts.shape[2] != m.nu:
@@ -322,14 +334,14 @@ def rollout(sys: S.System, state: State, acts, n_frames: int,
   xp = xr = xa = xv = None
   if frames:
     xp, xr, xa, xv = _frames(m, n, m.device)
-  status = torch.zeros(n, dtype=torch.int32, device=m.device)
+  status = torch.empty(n, dtype=torch.int32, device=m.device)
   lib = _lib.load()
   s = ctypes.c_void_p(stream) if stream is not None else _stream()
-  _lib.check(lib.bgx_rollout(m.handle, n, T, int(n_frames), _lib.ptr(q),
-                             _lib.ptr(qd), _lib.ptr(acts) if m.nu else None,
-                             n * m.nu, _lib.ptr(qt), _lib.ptr(qdt),
-                             _lib.ptr(xp), _lib.ptr(xr), _lib.ptr(xa),
-                             _lib.ptr(xv), _lib.ptr(status), s))
+  _lib.check(lib.bgx_rollout_from(m.handle, n, T, int(n_frames), _lib.ptr(q_in),
+                                  _lib.ptr(qd_in), _lib.ptr(q), _lib.ptr(qd),
+                                  _lib.ptr(acts) if m.nu else None, n * m.nu, _lib.ptr(qt),
+                                  _lib.ptr(qdt), _lib.ptr(xp), _lib.ptr(xr), _lib.ptr(xa),
+                                  _lib.ptr(xv), _lib.ptr(status), s))
   st = State(q=q, qd=qd,
              x=Transform(xp, xr) if frames else None,
              xd=Motion(xa, xv) if frames else None, status=status)
@@ -364,17 +376,17 @@ class _RolloutFn(torch.autograd.Function):
   @staticmethod
   def forward(ctx, q0, qd0, acts, m, n_frames, ckpt_every, min_workspace):
     n, T = q0.shape[0], acts.shape[0]
-    q = q0.detach().contiguous().clone()
-    qd = qd0.detach().contiguous().clone()
+    q_in, qd_in, q, qd = _state_io(q0.detach(), qd0.detach())
     a = acts.detach().contiguous()
     qt = torch.empty(T, n, m.nq, device=m.device)
     qdt = torch.empty(T, n, m.nv, device=m.device)
-    status = torch.zeros(n, dtype=torch.int32, device=m.device)
+    status = torch.empty(n, dtype=torch.int32, device=m.device)
     lib = _lib.load()
-    _lib.check(lib.bgx_rollout(m.handle, n, T, int(n_frames), _lib.ptr(q), _lib.ptr(qd),
-                               _lib.ptr(a) if m.nu else None, n * m.nu, _lib.ptr(qt),
-                               _lib.ptr(qdt), None, None, None, None, _lib.ptr(status),
-                               _stream()))
+    _lib.check(lib.bgx_rollout_from(m.handle, n, T, int(n_frames), _lib.ptr(q_in),
+                                    _lib.ptr(qd_in), _lib.ptr(q), _lib.ptr(qd),
+                                    _lib.ptr(a) if m.nu else None, n * m.nu, _lib.ptr(qt),
+                                    _lib.ptr(qdt), None, None, None, None, _lib.ptr(status),
+                                    _stream()))
     idx = list(range(ckpt_every - 1, T - 1, ckpt_every))
     ckq = torch.cat([q0.detach()[None].contiguous(), qt[idx]], 0).contiguous()
     ckqd = torch.cat([qd0.detach()[None].contiguous(), qdt[idx]], 0).contiguous()

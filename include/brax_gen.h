@@ -144,6 +144,19 @@ int bgx_rollout(const bgx_model* model, int32_t n_envs, int32_t n_steps,
                 float* x_pos, float* x_rot, float* xd_ang, float* xd_vel,
                 int32_t* status, void* stream);
 
+/* bgx_rollout from a state that the caller keeps: q_in and qd_in are read, q
+ * and qd (other arrays) receive the final state. */
+int bgx_rollout_from(const bgx_model* model, int32_t n_envs, int32_t n_steps,
+                     int32_t n_frames, const float* q_in, const float* qd_in, float* q,
+                     float* qd, const float* act, int64_t act_step_stride, float* q_traj,
+                     float* qd_traj, float* x_pos, float* x_rot, float* xd_ang,
+                     float* xd_vel, int32_t* status, void* stream);
+
+/* bgx_init, with copies of q_in and qd_in into q and qd. */
+int bgx_init_copy(const bgx_model* model, int32_t n_envs, const float* q_in,
+                  const float* qd_in, float* q, float* qd, float* x_pos, float* x_rot,
+                  float* xd_ang, float* xd_vel, void* stream);
+
 /* Every contact candidate of the states q (N, NQ), as the reference's
  * debug contact output (brax/generalized/pipeline.py:58-59, 91-92; MJX plane
  * collisions, brax/contact.py:28-67): dist (N, C), pos (N, C, 3) and frame
