@@ -19,6 +19,7 @@
 #include "bgx_launch.h"
 #include "bgx_mtree.h"
 #include "bgx_star.h"
+#include "bgx_star_adj.h"
 #include "bgx_step.h"
 
 namespace bgx {
@@ -453,6 +454,43 @@ constexpr bool star_tree() {
   else return star_ok<T>();
 }
 
+// Stage B, a lane per leg: blocks of STAR_ENVS envs, coordinate-major, then
+// one thread per env for the qd coordinates (as in k_adj_b, whose time per
+// substep it had been: 77 -> 24 us for 1,024 quadrupeds off the ground, 92 ->
+// 47 for 2,048, 104 -> 83 for 4,096).
+template <class T>
+__global__ __launch_bounds__(WAVE) void k_star_b(AdjLaunch a) {
+  constexpr int NQ = T::NQ, NV = T::NV, NU = T::NU, ND = NQ + NV;
+  __shared__ float lds[T::SIZE];
+  const int eb = (a.n + STAR_ENVS - 1) / STAR_ENVS;  // blocks of a coordinate
+  const int dir = (int)blockIdx.x / eb;
+  if (dir >= NQ) {
+    const int env = ((int)blockIdx.x - NQ * eb) * WAVE + (int)threadIdx.x;
+    if (env >= a.n) return;
+    float act[NU > 0 ? NU : 1], gqd[NV];
+#pragma unroll
+    for (int k = 0; k < NU; ++k) act[k] = a.act ? a.act[(long long)env * NU + k] : 0.f;
+    adjoint_b_qd_all<T>(a.M, a.q + (long long)env * NQ, a.qd + (long long)env * NV, act,
+                        RecPtr{a.rec + env, a.n}, gqd);
+#pragma unroll
+    for (int j = 0; j < NV; ++j) a.adj[(long long)env * ND + NQ + j] = gqd[j];
+    return;
+  }
+  const int b = threadIdx.x % STAR_LEGS;
+  const int env = ((int)blockIdx.x - dir * eb) * STAR_ENVS + (int)threadIdx.x / STAR_LEGS;
+  const int ec = env < a.n ? env : a.n - 1;
+  const RecPtr rec{a.rec + ec, a.n};
+  float g;
+  if (dir < 2) {  // xy_invariant: only the position update moves
+    g = rec[AdjRec<T>::GQ1 + dir];
+  } else {
+    star_stage<T>(a.M, lds);
+    g = star_adjoint_q<T>(lds, b, a.q + (long long)ec * NQ, a.qd + (long long)ec * NV,
+                          a.act ? a.act + (long long)ec * NU : nullptr, rec, dir);
+  }
+  if (env < a.n && b == 0) a.adj[(long long)env * ND + dir] = g;
+}
+
 // a batch launch of the rollout kernel: a persistent grid of `grid`
 // one-wavefront workgroups (a.items set)
 template <class T>
@@ -580,9 +618,15 @@ struct Ops {
   }
   static hipError_t adj_b(const AdjLaunch& a, hipStream_t s) {
     // NQ q coordinates, then the qd reverse pass
-    const long long threads = (long long)(a.n + WAVE - 1) / WAVE * WAVE * (T::NQ + 1);
-    hipLaunchKernelGGL(k_adj_b<T>, dim3((unsigned)((threads + WAVE - 1) / WAVE)), dim3(WAVE),
-                       0, s, a);
+    if constexpr (star_ok<T>()) {
+      const long long blocks = (long long)T::NQ * ((a.n + STAR_ENVS - 1) / STAR_ENVS) +
+                               (a.n + WAVE - 1) / WAVE;
+      hipLaunchKernelGGL(k_star_b<T>, dim3((unsigned)blocks), dim3(WAVE), 0, s, a);
+    } else {
+      const long long threads = (long long)(a.n + WAVE - 1) / WAVE * WAVE * (T::NQ + 1);
+      hipLaunchKernelGGL(k_adj_b<T>, dim3((unsigned)((threads + WAVE - 1) / WAVE)), dim3(WAVE),
+                         0, s, a);
+    }
     return hipGetLastError();
   }
   static hipError_t frames_vjp(const FramesVjp& a, hipStream_t s) {

@@ -159,6 +159,20 @@ BGX_D int star_act_of_leg(int b, int k) {
                 star_act<T>(6 + 3 * K + k));
 }
 
+// the limit row of leg b's k-th hinge
+template <class T>
+constexpr int star_lim_row(int d) {
+  for (int i = 0; i < T::NLIM; ++i)
+    if (T::LIM_D[i] == d) return i;
+  return 0;
+}
+template <class T>
+BGX_D int star_lim_of_leg(int b, int k) {
+  constexpr int K = Star<T>::K;
+  return by_leg(b, star_lim_row<T>(6 + k), star_lim_row<T>(6 + K + k),
+                star_lim_row<T>(6 + 2 * K + k), star_lim_row<T>(6 + 3 * K + k));
+}
+
 template <class T>
 struct StarState {
   static constexpr int K = Star<T>::K;
@@ -197,39 +211,40 @@ BGX_D void star_store_qd(const StarState<T>& s, int b, float* qdp) {
 
 // world frames of the root and of this lane's leg (kinematics.py:31-108);
 // XD: also the frames' velocities
-template <class T, bool XD>
-BGX_D void star_frames(const float* ml, int b, const StarState<T>& s, V3& xp0, Q4& xr0, V3* xp,
-                       Q4* xr, V3* xa0, V3* xa, V3* xv) {
+template <class T, bool XD, class S>
+BGX_D void star_frames(const float* ml, int b, const S* rq, const S* q, const float* rv,
+                       const float* qd, V3T<S>& xp0, Q4T<S>& xr0, V3T<S>* xp, Q4T<S>* xr,
+                       V3T<S>* xa0, V3T<S>* xa, V3T<S>* xv) {
   constexpr int K = Star<T>::K;
   const float* lk = ml + T::OFF_LINK;
   {
-    V3 p = v3(s.rq[0], s.rq[1], s.rq[2]);
-    const Q4 r{s.rq[3], s.rq[4], s.rq[5], s.rq[6]};
-    const V3 jpos = ldv3(lk + LK_JPOS);
+    V3T<S> p{rq[0], rq[1], rq[2]};
+    const Q4T<S> r{rq[3], rq[4], rq[5], rq[6]};
+    const V3T<S> jpos = lift3<S>(ldv3(lk + LK_JPOS));
     p = (p + jpos) - rotate(jpos, r);
-    const Q4 trot = ldq4(lk + LK_TROT);
-    xp0 = ldv3(lk + LK_TPOS) + rotate(p, trot);
+    const Q4T<S> trot = lift4<S>(ldq4(lk + LK_TROT));
+    xp0 = lift3<S>(ldv3(lk + LK_TPOS)) + rotate(p, trot);
     xr0 = qmul(trot, r);
   }
-  if constexpr (XD) *xa0 = rotate(v3(s.rv[3], s.rv[4], s.rv[5]), xr0);
+  if constexpr (XD) *xa0 = rotate(lift3<S>(v3(rv[3], rv[4], rv[5])), xr0);
   lk += LINK_STRIDE * (1 + b * K);
   const float* df = ml + T::OFF_DOF + DOF_STRIDE * (6 + b * K);
 #pragma unroll
   for (int k = 0; k < K; ++k, lk += LINK_STRIDE, df += DOF_STRIDE) {
-    const V3 ang = ldv3(df + DF_ANG);
-    const Q4 rk = qnormalize(qrot_axis(ang, s.q[k]));
-    const V3 jpos = ldv3(lk + LK_JPOS);
-    const Q4 trot = ldq4(lk + LK_TROT);
-    const V3 p = ldv3(lk + LK_TPOS) + rotate(jpos - rotate(jpos, rk), trot);
-    const V3 pp = k == 0 ? xp0 : xp[k - 1];
-    const Q4 pr = k == 0 ? xr0 : xr[k - 1];
+    const V3T<S> ang = lift3<S>(ldv3(df + DF_ANG));
+    const Q4T<S> rk = qnormalize(qrot_axis(ang, q[k]));
+    const V3T<S> jpos = lift3<S>(ldv3(lk + LK_JPOS));
+    const Q4T<S> trot = lift4<S>(ldq4(lk + LK_TROT));
+    const V3T<S> p = lift3<S>(ldv3(lk + LK_TPOS)) + rotate(jpos - rotate(jpos, rk), trot);
+    const V3T<S> pp = k == 0 ? xp0 : xp[k - 1];
+    const Q4T<S> pr = k == 0 ? xr0 : xr[k - 1];
     xp[k] = pp + rotate(p, pr);
     xr[k] = qmul(pr, qmul(trot, rk));
     if constexpr (XD) {
-      const V3 pa = k == 0 ? *xa0 : xa[k - 1];
-      const V3 pv = k == 0 ? v3(s.rv[0], s.rv[1], s.rv[2]) : xv[k - 1];
+      const V3T<S> pa = k == 0 ? *xa0 : xa[k - 1];
+      const V3T<S> pv = k == 0 ? lift3<S>(v3(rv[0], rv[1], rv[2])) : xv[k - 1];
       xv[k] = pv + cross(pa, xp[k] - pp);
-      xa[k] = pa + rotate(ang * s.qd[k], xr[k]);
+      xa[k] = pa + rotate(ang * qd[k], xr[k]);
     }
   }
   xr0 = qnormalize(xr0);
@@ -239,24 +254,28 @@ BGX_D void star_frames(const float* ml, int b, const StarState<T>& s, V3& xp0, Q
 
 // mass-weighted COM offset and rotational inertia of one link about rc
 // (dynamics.py:44-55)
-BGX_D void star_inertia(const float* lk, V3 xp, Q4 xr, V3 rc, V3& cc, Sym3& ci) {
-  const V3 p = (xp + rotate(ldv3(lk + LK_IPOS), xr)) - rc;
+template <class S>
+BGX_D void star_inertia(const float* lk, V3T<S> xp, Q4T<S> xr, V3T<S> rc, V3T<S>& cc,
+                        Sym3T<S>& ci) {
+  const V3T<S> p = (xp + rotate(lift3<S>(ldv3(lk + LK_IPOS)), xr)) - rc;
   const float m = lk[LK_MASS];
-  float R[3][3], RI[3][3];
-  quat_to_3x3(qmul(xr, ldq4(lk + LK_IROT)), R);
-  const Sym3 I0 = ldsym(lk + LK_I);
+  S R[3][3], RI[3][3];
+  quat_to_3x3(qmul(xr, lift4<S>(ldq4(lk + LK_IROT))), R);
+  const float* i0 = lk + LK_I;
+  const Sym3T<S> I0{lift<S>(i0[0]), lift<S>(i0[1]), lift<S>(i0[2]),
+                    lift<S>(i0[3]), lift<S>(i0[4]), lift<S>(i0[5])};
 #pragma unroll
   for (int i = 0; i < 3; ++i) {
-    const V3 c = symmul(I0, V3{R[i][0], R[i][1], R[i][2]});
+    const V3T<S> c = symmul(I0, V3T<S>{R[i][0], R[i][1], R[i][2]});
     RI[i][0] = c.x, RI[i][1] = c.y, RI[i][2] = c.z;
   }
   auto rir = [&](int i, int j) {
     return RI[i][0] * R[j][0] + RI[i][1] * R[j][1] + RI[i][2] * R[j][2];
   };
-  const float pp = dot(p, p);
-  ci = Sym3{rir(0, 0) + (pp - p.x * p.x) * m, rir(1, 1) + (pp - p.y * p.y) * m,
-            rir(2, 2) + (pp - p.z * p.z) * m, rir(0, 1) - p.x * p.y * m,
-            rir(0, 2) - p.x * p.z * m, rir(1, 2) - p.y * p.z * m};
+  const S pp = dot(p, p);
+  ci = Sym3T<S>{rir(0, 0) + (pp - p.x * p.x) * m, rir(1, 1) + (pp - p.y * p.y) * m,
+                rir(2, 2) + (pp - p.z * p.z) * m, rir(0, 1) - p.x * p.y * m,
+                rir(0, 2) - p.x * p.z * m, rir(1, 2) - p.y * p.z * m};
   cc = p * m;
 }
 
@@ -377,7 +396,8 @@ BGX_D int star_substep(float* ml, int b, StarState<T>& s, const float* act,
 
   V3 xp0, xp[K];
   Q4 xr0, xr[K];
-  star_frames<T, false>(ml, b, s, xp0, xr0, xp, xr, nullptr, nullptr, nullptr);
+  star_frames<T, false, float>(ml, b, s.rq, s.q, nullptr, nullptr, xp0, xr0, xp, xr, nullptr,
+                               nullptr, nullptr);
 
   // ---- root COM (dynamics.py:37-43), cinr (:44-55)
   const float m0 = lk0[LK_MASS];
@@ -919,7 +939,7 @@ BGX_ITEM void star_write_frames(const Launch& a, long long env, int b, float* ld
   const float* ml = star_lds(lds);
   V3 xp0, xp[K], xa0, xa[K], xv[K];
   Q4 xr0, xr[K];
-  star_frames<T, true>(ml, b, s, xp0, xr0, xp, xr, &xa0, xa, xv);
+  star_frames<T, true, float>(ml, b, s.rq, s.q, s.rv, s.qd, xp0, xr0, xp, xr, &xa0, xa, xv);
   if (!live) return;
   const long long o = env * T::L, ol = o + 1 + b * K;
   auto put3 = [&](float* base, V3 root, const V3* leg) {
