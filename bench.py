@@ -185,21 +185,24 @@ def forward_bench(args, name):
   q_init = torch.tensor(q0, device=dev)
   qd_init = torch.tensor(qd0, device=dev)
   epw, kc = 64, None
+  from brax_amd.generalized import autotune
   if args.lanes:
-    from brax_amd.generalized import autotune
     autotune.set_launch(m, autotune.LANES, args.lanes)
   lanes = lib.bgx_model_get_launch(m.handle, 3)
   kernel = {1: "k_rollout", 4: "k_star"}.get(lanes, "k_mtree")
+  if not args.no_tune:
+    # the tile trades occupancy against slow-path substeps, which grow as
+    # the envs settle onto the floor: time it over the timed steps (up to 20);
+    # 0: a multi-lane kernel was faster
+    kc = autotune.tune_tile(sys_, q_init, qd_init, acts[:min(K, 20)], N_FRAMES)
+    if lanes == 4 and kc:
+      lanes, kernel = 1, "k_rollout"
   if lanes > 1:
     # a multi-lane kernel's workgroup is one wavefront of 64 / lanes envs,
     # and it keeps one contact row per candidate lane (no LDS tile)
-    epw = 64 // lanes
+    epw, kc = 64 // lanes, None
   elif not args.no_tune:
-    from brax_amd.generalized import autotune
     epw = autotune.tune_step(sys_, q_init, qd_init, acts[:2], N_FRAMES)
-    # the tile trades occupancy against slow-path substeps, which grow as
-    # the envs settle onto the floor: time it over the timed steps (up to 20)
-    kc = autotune.tune_tile(sys_, q_init, qd_init, acts[:min(K, 20)], N_FRAMES)
   q = q_init.clone()
   qd = qd_init.clone()
   status = torch.zeros(n, dtype=torch.int32, device=dev)

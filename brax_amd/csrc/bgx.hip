@@ -197,6 +197,22 @@ int bgx_model_get_launch(const bgx_model* m, int kernels) {
   return m->epw[kernels] ? m->epw[kernels] : bgx::WAVE;
 }
 
+// Lanes per env of a rollout of n envs over n_sub substeps (Launch::lanes).
+// A lane per leg needs four wavefronts for 64 envs, each alone on its SIMD:
+// up to two for every SIMD (32,768 envs) it is faster at any contact load
+// (quadrupeds settled on the floor: 86 us a substep against 114 with one
+// thread per env).  At 65,536 it is as fast over the first substeps from a
+// standing start (141 us against 146), but long rollouts settle, the solver
+// grows, and one thread per env takes over: 171 us a substep against 110 over
+// 1,000 env steps.
+static int rollout_lanes(const bgx_model* m, int64_t n, int64_t n_sub) {
+  constexpr int64_t kStarEnvs = 2 * 16 * 1024, kStarSubsteps = 25;
+  if (m->lanes == 0 && kOps[m->topo]->mlanes == bgx::STAR_LEGS && n > kStarEnvs &&
+      n_sub > kStarSubsteps)
+    return 1;
+  return m->lanes;
+}
+
 static int launch(const bgx_model* m, bool init_only, bgx::Launch a, void* stream) {
   if (!m) return fail(BGX_ERR_ARG, "model is null");
   if (!valid_topo(m->topo)) return fail(BGX_ERR_TOPOLOGY, "unknown topology id");
@@ -209,7 +225,7 @@ static int launch(const bgx_model* m, bool init_only, bgx::Launch a, void* strea
   a.M = m->table;
   a.epw = m->epw[BGX_KERNELS_STEP];
   a.kc = m->kc;
-  a.lanes = m->lanes;
+  a.lanes = rollout_lanes(m, a.n, (int64_t)a.n_steps * a.n_frames);
   const bgx::TopoOps* ops = kOps[m->topo];
   a.q_step = (long long)a.n * ops->dims[1], a.qd_step = (long long)a.n * ops->dims[2];
   if ((a.q_traj || a.qd_traj) && a.n_seg > 1)
@@ -525,7 +541,7 @@ int adjoint_part(const bgx_model* m, int n, int env0, int nh, int n_steps, int n
     f.status = status ? status + env0 : nullptr, f.status_or = 1;
     f.epw = m->epw[BGX_KERNELS_ADJOINT];
     f.kc = m->kc;  // the forward's tile and kernel: the recompute repeats its states
-    f.lanes = m->lanes;
+    f.lanes = rollout_lanes(m, n, (int64_t)n_steps * n_frames);
     if ((rc = check_hip(ops->rollout(f, s), "recompute launch"))) return rc;
     for (int seg = seg_hi; seg >= seg_lo; --seg) {
       const int s0 = seg * ckpt_every;
@@ -732,7 +748,7 @@ int bgx_batch_create(int32_t n_models, const bgx_model* const* models,
     kernel_topo = md->topo;
   }
   if (kernel_topo < 0) kernel_topo = chain_topo;  // chains only (or empty)
-  // work items: 64 tree envs, or one wavefront of chains (64 / G envs)
+  // work items: one wavefront of tree envs or of chains (64 / lanes per env)
   std::vector<bgx::BatchItem> items;
   std::vector<int> rank;  // ordering key: tree items first, then wider chains
   std::vector<int64_t> table_off(n_models), table_len(n_models);

@@ -21,6 +21,9 @@
 //    lanes (an inactive candidate's rows are zero, which leaves every
 //    projected-gradient iterate as if they were dropped, constraint.py:174),
 //    and the solver's sums are butterfly reductions over the group.
+// LDS issue and latency bound it: 239 -> 159 us a substep for 16,384 humanoids
+// off the ground, 254 -> 150 us for 1,000 on their feet, since the rows of the
+// mass matrix stay in registers and pairs are read as float4s.
 // The topology must be one tree whose root link (link 0) has the free joint
 // or a hinge stack, without sphere / capsule pairs, with at most one
 // actuator per dof acting on that dof's own coordinate (codegen checks).

@@ -102,8 +102,8 @@ def tune_tile(sys, q: torch.Tensor, qd: torch.Tensor, acts: torch.Tensor, n_fram
   take more LDS per env (fewer workgroups per compute unit); which wins
   depends on the batch's contact counts, which change as the envs settle,
   so acts should span the horizon of interest (a two-step window from
-  standing starts picks too few slots).  Where several lanes per env are the
-  default, that kernel is timed too: choice 0.  Returns the choice, which is
+  standing starts picks too few slots).  Where a lane per leg is the default,
+  that kernel is timed too: choice 0.  Returns the choice, which is
   set on the model."""
   m = pipeline.device_model(sys, q.device)
   n = q.shape[0]
@@ -112,8 +112,10 @@ def tune_tile(sys, q: torch.Tensor, qd: torch.Tensor, acts: torch.Tensor, n_fram
     set_launch(m, TILE, _CACHE[key])
     return _CACHE[key]
   cands = tiles(sys, q.device)
-  if get_launch(m, LANES) > 1:
-    cands = (0,) + cands  # the multi-lane kernel, which has no tile
+  if get_launch(m, LANES) == 4:
+    cands = (0,) + cands  # the lane-per-leg kernel, which has no tile
+  if cands[0] == 0 and len(cands) == 2:
+    cands = cands[:1]  # one tile, beside the default: nothing to choose
   if len(cands) == 1:
     set_launch(m, TILE, cands[0])
     _CACHE[key] = cands[0]

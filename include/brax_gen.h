@@ -98,8 +98,9 @@ int bgx_model_topology(const bgx_model* model);
  * where the topology is compiled with a multi-lane kernel) runs an env on a
  * group of lanes: 4 for a free root with four equal legs (a lane per leg),
  * a lane per dof for other large trees.  The two agree within rounding; the
- * getter returns the width.  Choosing an LDS tile runs a four-legged
- * topology at one thread per env. */
+ * getter returns the width.  A four-legged topology runs at one thread per
+ * env all the same where an LDS tile is chosen, and in rollouts of more than
+ * 32,768 envs over more than 25 substeps. */
 #define BGX_KERNELS_LANES 3
 /* kernels = BGX_KERNELS_ADJOINT_PARTS splits bgx_rollout_adjoint's backward
  * pass into that many parts of whole envs (1-4; 0 = one), each on its own
