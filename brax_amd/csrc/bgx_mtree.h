@@ -21,9 +21,10 @@
 //    lanes (an inactive candidate's rows are zero, which leaves every
 //    projected-gradient iterate as if they were dropped, constraint.py:174),
 //    and the solver's sums are butterfly reductions over the group.
-// LDS issue and latency bound it: 239 -> 159 us a substep for 16,384 humanoids
-// off the ground, 254 -> 150 us for 1,000 on their feet, since the rows of the
-// mass matrix stay in registers and pairs are read as float4s.
+// LDS issue and latency bound it.  With the rows of the mass matrix in LDS,
+// then in registers with pairs read as float4s: ten substeps of 16,384
+// humanoids off the ground 2,422 -> 1,595 us, one of 1,000 on their feet with
+// its frames 274 -> 164 us, the results bit for bit the same.
 // The topology must be one tree whose root link (link 0) has the free joint
 // or a hinge stack, without sphere / capsule pairs, with at most one
 // actuator per dof acting on that dof's own coordinate (codegen checks).
@@ -166,6 +167,16 @@ BGX_D Q4 ld4l(const float* p) { return Q4{p[0], p[1], p[2], p[3]}; }
 // solver's loops would spill)
 BGX_D float masked(float x, unsigned m, int k) {
   return __builtin_bit_cast(float, __builtin_bit_cast(int, x) & ((int)(m << (31 - k)) >> 31));
+}
+// a . b with its roundings spelled out (fdot rounds y's product, fdotx x's).
+// Which product the compiler rounds depends on the code around it; the two
+// entries of M that mirror each other, computed on two lanes, must be the same
+// bits, and the line search decides ties by the last bits of the contact rows.
+BGX_D float fdot(V3 a, V3 b) {
+  return __builtin_fmaf(a.z, b.z, __builtin_fmaf(a.x, b.x, a.y * b.y));
+}
+BGX_D float fdotx(V3 a, V3 b) {
+  return __builtin_fmaf(a.z, b.z, __builtin_fmaf(a.y, b.y, a.x * b.x));
 }
 // 16-byte aligned LDS: a pair's half, and row j / 4 of a padded vector
 BGX_D V3 ld3a(const float* p) {
@@ -573,16 +584,16 @@ BGX_D void mtree_substep(const float* __restrict__ M, MLane<T>& s, const float* 
   {
     const unsigned danc = d >= 0 ? T::DANC[d] : 0u;
     const float arm = d >= 0 ? dof_rec<T>(M, d)[DF_ARMATURE] : 1.f;
+    const float diag = (fdotx(cv, Fv) + fdot(ca, Fa)) + arm;
 #pragma unroll
     for (int j = 0; j < NV; ++j) {
       const float* cf = lds + MT::CDF + 8 * j;
       const float* fs = lds + MT::FS + 8 * j;
-      const float lower = dot(ld3a(cf + 4), Fv) + dot(ld3a(cf), Fa);
-      const float upper = dot(cv, ld3a(fs + 4)) + dot(ca, ld3a(fs));
+      const float lower = fdot(ld3a(cf + 4), Fv) + fdot(ld3a(cf), Fa);
+      const float upper = fdot(cv, ld3a(fs + 4)) + fdot(ca, ld3a(fs));
       const bool in_lower = j < d && ((danc >> j) & 1u);
       const bool in_upper = j > d && ((T::DANC[j] >> (d >= 0 ? d : 0)) & 1u);
-      mrow[j] = j == d ? (dot(cv, Fv) + dot(ca, Fa)) + arm
-                       : (in_lower ? lower : (in_upper ? upper : 0.f));
+      mrow[j] = j == d ? diag : (in_lower ? lower : (in_upper ? upper : 0.f));
       // four columns' reads in flight, not all of them
       if (j % 4 == 3) asm volatile("" ::: "memory");
     }
@@ -678,8 +689,8 @@ BGX_D void mtree_substep(const float* __restrict__ M, MLane<T>& s, const float* 
       const float* fq = lds + MT::LB + 6 * cl;
       const V3 vu = uv + cross(ua, r);
       const V3 vq = ld3l(fq + 3) + cross(ld3l(fq), r);
-      const float e0u = dot(d0, vu), e1u = dot(d1, vu), e2u = dot(d2, vu);
-      const float e0q = dot(d0, vq), e1q = dot(d1, vq), e2q = dot(d2, vq);
+      const float e0u = fdotx(d0, vu), e1u = fdotx(d1, vu), e2u = fdotx(d2, vu);
+      const float e0q = fdot(d0, vq), e1q = fdot(d1, vq), e2q = fdot(d2, vq);
       sb[0] = (e0u + e1u) + (bq * (e0q + e1q) + kt);
       sb[1] = (e0u - e1u) + (bq * (e0q - e1q) + kt);
       sb[2] = (e0u + e2u) + (bq * (e0q + e2q) + kt);
@@ -742,7 +753,7 @@ BGX_D void mtree_substep(const float* __restrict__ M, MLane<T>& s, const float* 
       V3 wa, wv;
       path_vel(MT::ZW, wa, wv);
       const V3 vp = wv + cross(wa, r);
-      const float e0 = dot(d0, vp), e1 = dot(d1, vp), e2 = dot(d2, vp);
+      const float e0 = fdotx(d0, vp), e1 = fdotx(d1, vp), e2 = fdotx(d2, vp);
       out[0] = active ? e0 + e1 + sdiag * in[0] : 0.f;
       out[1] = active ? e0 - e1 + sdiag * in[1] : 0.f;
       out[2] = active ? e0 + e2 + sdiag * in[2] : 0.f;
@@ -775,6 +786,11 @@ BGX_D void mtree_substep(const float* __restrict__ M, MLane<T>& s, const float* 
         if (running) Rr[k] = active ? o[k] + sb[k] : 0.f;
       if (running) rl = ol + lb;
     }
+    float fy = 0.f;
+#pragma unroll
+    for (int k = 0; k < 4; ++k) fy += active ? 0.5f * Rr[k] * Rr[k] : 0.f;
+    fy += has_l ? 0.5f * rl * rl : 0.f;
+    fy = gsum<G>(fy);
     {
       apply_a(Rr, rl, o, ol);
 #pragma unroll
@@ -782,10 +798,11 @@ BGX_D void mtree_substep(const float* __restrict__ M, MLane<T>& s, const float* 
         if (running) Gr[k] = o[k];
       if (running) gl = ol;
     }
-    // line search over x+ = relu(y - eta g), the test in terms of A d,
-    // d = x+ - y (bgx_star.h): f(x+) - f(y) > g.d + |d|^2 / (2 eta) is
-    // |A d|^2 / 2 > |d|^2 / (2 eta), where rounding decides no step.  R
-    // becomes A d.
+    // line search: trial x+ = relu(y - eta g), residual into r.  The test is
+    // the taped substep's (bgx_step.h), on f.  Written as |A d|^2 against
+    // |d|^2 / eta, d = x+ - y, it is the same only in exact arithmetic: at a
+    // tie the two round apart, and the gradient would follow another step
+    // than the states.
     bool cond = running;
     for (int ls = 0; ls <= maxls; ++ls) {
       if (!wave_any(cond)) break;
@@ -793,26 +810,34 @@ BGX_D void mtree_substep(const float* __restrict__ M, MLane<T>& s, const float* 
       const float e_ = eta;
       float in[4], in_l;
 #pragma unroll
-      for (int k = 0; k < 4; ++k) in[k] = fmaxf(Y[k] - e_ * Gr[k], 0.f) - Y[k];
-      in_l = fmaxf(yl - e_ * gl, 0.f) - yl;
+      for (int k = 0; k < 4; ++k) in[k] = fmaxf(Y[k] - e_ * Gr[k], 0.f);
+      in_l = fmaxf(yl - e_ * gl, 0.f);
       apply_a(in, in_l, o, ol);
-      float ad = 0.f, dd = 0.f;
+      float fx = 0.f, dg = 0.f, dd = 0.f;
 #pragma unroll
       for (int k = 0; k < 4; ++k) {
-        if (cond) Rr[k] = o[k];
-        ad += active ? o[k] * o[k] : 0.f;
-        dd += active ? in[k] * in[k] : 0.f;
+        const float rv = o[k] + sb[k];
+        if (cond) Rr[k] = rv;
+        const float df = in[k] - Y[k];
+        fx += active ? 0.5f * rv * rv : 0.f;
+        dg += active ? df * Gr[k] : 0.f;
+        dd += active ? df * df : 0.f;
       }
-      if (cond) rl = ol;
-      ad += has_l ? ol * ol : 0.f;
-      dd += has_l ? in_l * in_l : 0.f;
-      ad = gsum<G>(ad), dd = gsum<G>(dd);
+      {
+        const float rv = ol + lb;
+        if (cond) rl = rv;
+        const float df = in_l - yl;
+        fx += has_l ? 0.5f * rv * rv : 0.f;
+        dg += has_l ? df * gl : 0.f;
+        dd += has_l ? df * df : 0.f;
+      }
+      fx = gsum<G>(fx), dg = gsum<G>(dg), dd = gsum<G>(dd);
       if (cond) {
         trials += 1;
-        cond = e_ * (0.5f * ad) > 0.5f * dd + lseps;
+        cond = e_ * (fx - fy) > e_ * dg + 0.5f * dd + lseps;
       }
     }
-    // error at x+: |relu(x+ - grad f(x+)) - x+|, grad f(x+) = g + A^T A d
+    // error at x+: |relu(x+ - grad f(x+)) - x+| with grad = A^T (A x+ + b)
     const float e_ = eta;
     apply_a(Rr, rl, o, ol);
     float e2 = 0.f;
@@ -820,12 +845,12 @@ BGX_D void mtree_substep(const float* __restrict__ M, MLane<T>& s, const float* 
 #pragma unroll
     for (int k = 0; k < 4; ++k) {
       xp[k] = fmaxf(Y[k] - e_ * Gr[k], 0.f);
-      const float dv = fmaxf(xp[k] - (Gr[k] + o[k]), 0.f) - xp[k];
+      const float dv = fmaxf(xp[k] - o[k], 0.f) - xp[k];
       e2 += active ? dv * dv : 0.f;
     }
     xpl = fmaxf(yl - e_ * gl, 0.f);
     {
-      const float dv = fmaxf(xpl - (gl + ol), 0.f) - xpl;
+      const float dv = fmaxf(xpl - ol, 0.f) - xpl;
       e2 += has_l ? dv * dv : 0.f;
     }
     e2 = gsum<G>(e2);
