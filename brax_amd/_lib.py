@@ -46,6 +46,8 @@ SIGNATURES = {
     "bgx_init_copy": (c_int, [c_vp, c_i32] + [c_vp] * 9),
     "bgx_rollout_from": (c_int, [c_vp, c_i32, c_i32, c_i32, c_vp, c_vp, c_vp, c_vp, c_vp, c_i64,
                                  c_vp, c_vp, c_vp, c_vp, c_vp, c_vp, c_vp, c_vp]),
+    "bgx_rollout_primal": (c_int, [c_vp, c_i32, c_i32, c_i32, c_vp, c_vp, c_vp, c_vp, c_vp, c_i64,
+                                   c_vp, c_vp, c_vp, c_vp, c_vp, c_vp, c_vp, c_vp]),
     "bgx_contacts": (c_int, [c_vp, c_i32, c_vp, c_vp, c_vp, c_vp, c_vp]),
     "bgx_step_probe": (c_int, [c_vp, c_i32, c_i32, c_vp, c_vp, c_vp, c_vp,
                                c_vp]),

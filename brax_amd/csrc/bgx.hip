@@ -213,7 +213,17 @@ static int rollout_lanes(const bgx_model* m, int64_t n, int64_t n_sub) {
   return m->lanes;
 }
 
-static int launch(const bgx_model* m, bool init_only, bgx::Launch a, void* stream) {
+// Lanes per env of the states that the adjoint differentiates, forward and
+// recompute: where a lane per leg is the step's kernel, one thread per env,
+// the code that stage A1 tapes (bgx_step.h), so that the tape starts from and
+// arrives at the same bits.
+static int primal_lanes(const bgx_model* m) {
+  return kOps[m->topo]->mlanes == bgx::STAR_LEGS ? 1 : m->lanes;
+}
+
+enum class Run { INIT, STEP, PRIMAL };
+
+static int launch(const bgx_model* m, Run run, bgx::Launch a, void* stream) {
   if (!m) return fail(BGX_ERR_ARG, "model is null");
   if (!valid_topo(m->topo)) return fail(BGX_ERR_TOPOLOGY, "unknown topology id");
   if (a.n < 0) return fail(BGX_ERR_ARG, "negative env count");
@@ -225,13 +235,14 @@ static int launch(const bgx_model* m, bool init_only, bgx::Launch a, void* strea
   a.M = m->table;
   a.epw = m->epw[BGX_KERNELS_STEP];
   a.kc = m->kc;
-  a.lanes = rollout_lanes(m, a.n, (int64_t)a.n_steps * a.n_frames);
+  a.lanes = run == Run::PRIMAL ? primal_lanes(m)
+                               : rollout_lanes(m, a.n, (int64_t)a.n_steps * a.n_frames);
   const bgx::TopoOps* ops = kOps[m->topo];
   a.q_step = (long long)a.n * ops->dims[1], a.qd_step = (long long)a.n * ops->dims[2];
   if ((a.q_traj || a.qd_traj) && a.n_seg > 1)
     return fail(BGX_ERR_ARG, "trajectories of a multi-segment launch are not supported");
   hipStream_t s = static_cast<hipStream_t>(stream);
-  return check_hip(init_only ? ops->init(a, s) : ops->rollout(a, s), "kernel launch");
+  return check_hip(run == Run::INIT ? ops->init(a, s) : ops->rollout(a, s), "kernel launch");
 }
 
 int bgx_init(const bgx_model* m, int32_t n, const float* q, const float* qd, float* x_pos,
@@ -241,7 +252,7 @@ int bgx_init(const bgx_model* m, int32_t n, const float* q, const float* qd, flo
   a.q = const_cast<float*>(q);
   a.qd = const_cast<float*>(qd);
   a.x_pos = x_pos, a.x_rot = x_rot, a.xd_ang = xd_ang, a.xd_vel = xd_vel;
-  return launch(m, true, a, stream);
+  return launch(m, Run::INIT, a, stream);
 }
 
 int bgx_init_copy(const bgx_model* m, int32_t n, const float* q_in, const float* qd_in, float* q,
@@ -252,14 +263,14 @@ int bgx_init_copy(const bgx_model* m, int32_t n, const float* q_in, const float*
   a.n = n;
   a.q = q, a.qd = qd, a.q_in = q_in, a.qd_in = qd_in;
   a.x_pos = x_pos, a.x_rot = x_rot, a.xd_ang = xd_ang, a.xd_vel = xd_vel;
-  return launch(m, true, a, stream);
+  return launch(m, Run::INIT, a, stream);
 }
 
-int bgx_rollout_from(const bgx_model* m, int32_t n, int32_t n_steps, int32_t n_frames,
-                     const float* q_in, const float* qd_in, float* q, float* qd,
-                     const float* act, int64_t act_step_stride, float* q_traj, float* qd_traj,
-                     float* x_pos, float* x_rot, float* xd_ang, float* xd_vel, int32_t* status,
-                     void* stream) {
+static int rollout_from(const bgx_model* m, Run run, int32_t n, int32_t n_steps,
+                        int32_t n_frames, const float* q_in, const float* qd_in, float* q,
+                        float* qd, const float* act, int64_t act_step_stride, float* q_traj,
+                        float* qd_traj, float* x_pos, float* x_rot, float* xd_ang,
+                        float* xd_vel, int32_t* status, void* stream) {
   if (n > 0 && (!q_in || !qd_in)) return fail(BGX_ERR_ARG, "q/qd must be non-null");
   bgx::Launch a{};
   a.n = n, a.n_steps = n_steps, a.n_frames = n_frames;
@@ -268,7 +279,27 @@ int bgx_rollout_from(const bgx_model* m, int32_t n, int32_t n_steps, int32_t n_f
   a.q_traj = q_traj, a.qd_traj = qd_traj;
   a.x_pos = x_pos, a.x_rot = x_rot, a.xd_ang = xd_ang, a.xd_vel = xd_vel;
   a.status = status;
-  return launch(m, false, a, stream);
+  return launch(m, run, a, stream);
+}
+
+int bgx_rollout_from(const bgx_model* m, int32_t n, int32_t n_steps, int32_t n_frames,
+                     const float* q_in, const float* qd_in, float* q, float* qd,
+                     const float* act, int64_t act_step_stride, float* q_traj, float* qd_traj,
+                     float* x_pos, float* x_rot, float* xd_ang, float* xd_vel, int32_t* status,
+                     void* stream) {
+  return rollout_from(m, Run::STEP, n, n_steps, n_frames, q_in, qd_in, q, qd, act,
+                      act_step_stride, q_traj, qd_traj, x_pos, x_rot, xd_ang, xd_vel, status,
+                      stream);
+}
+
+int bgx_rollout_primal(const bgx_model* m, int32_t n, int32_t n_steps, int32_t n_frames,
+                       const float* q_in, const float* qd_in, float* q, float* qd,
+                       const float* act, int64_t act_step_stride, float* q_traj,
+                       float* qd_traj, float* x_pos, float* x_rot, float* xd_ang,
+                       float* xd_vel, int32_t* status, void* stream) {
+  return rollout_from(m, Run::PRIMAL, n, n_steps, n_frames, q_in, qd_in, q, qd, act,
+                      act_step_stride, q_traj, qd_traj, x_pos, x_rot, xd_ang, xd_vel, status,
+                      stream);
 }
 
 int bgx_step(const bgx_model* m, int32_t n, int32_t n_frames, float* q, float* qd,
@@ -279,7 +310,7 @@ int bgx_step(const bgx_model* m, int32_t n, int32_t n_frames, float* q, float* q
   a.q = q, a.qd = qd, a.act = act, a.act_stride = 0;
   a.x_pos = x_pos, a.x_rot = x_rot, a.xd_ang = xd_ang, a.xd_vel = xd_vel;
   a.status = status;
-  return launch(m, false, a, stream);
+  return launch(m, Run::STEP, a, stream);
 }
 
 int bgx_rollout(const bgx_model* m, int32_t n, int32_t n_steps, int32_t n_frames, float* q,
@@ -292,7 +323,7 @@ int bgx_rollout(const bgx_model* m, int32_t n, int32_t n_steps, int32_t n_frames
   a.q_traj = q_traj, a.qd_traj = qd_traj;
   a.x_pos = x_pos, a.x_rot = x_rot, a.xd_ang = xd_ang, a.xd_vel = xd_vel;
   a.status = status;
-  return launch(m, false, a, stream);
+  return launch(m, Run::STEP, a, stream);
 }
 
 int bgx_contacts(const bgx_model* m, int32_t n, const float* q, float* dist, float* pos,
@@ -336,7 +367,7 @@ int bgx_step_probe(const bgx_model* m, int32_t n, int32_t n_frames, float* q, fl
   a.n = n, a.n_steps = 1, a.n_frames = n_frames;
   a.q = q, a.qd = qd, a.act = act, a.act_stride = 0;
   a.probe = probe;
-  return launch(m, false, a, stream);
+  return launch(m, Run::STEP, a, stream);
 }
 
 // ---------------------------------------------------------------------------
@@ -540,8 +571,8 @@ int adjoint_part(const bgx_model* m, int n, int env0, int nh, int n_steps, int n
     f.sub_q = w.sub_q, f.sub_qd = w.sub_qd;
     f.status = status ? status + env0 : nullptr, f.status_or = 1;
     f.epw = m->epw[BGX_KERNELS_ADJOINT];
-    f.kc = m->kc;  // the forward's tile and kernel: the recompute repeats its states
-    f.lanes = rollout_lanes(m, n, (int64_t)n_steps * n_frames);
+    f.kc = m->kc;  // bgx_rollout_primal's tile and kernel: its states again
+    f.lanes = primal_lanes(m);
     if ((rc = check_hip(ops->rollout(f, s), "recompute launch"))) return rc;
     for (int seg = seg_hi; seg >= seg_lo; --seg) {
       const int s0 = seg * ckpt_every;

@@ -29,6 +29,7 @@
 
 #include "bgx_layout.h"
 #include "bgx_math.h"
+#include "bgx_star_shape.h"
 
 namespace bgx {
 
@@ -1393,11 +1394,43 @@ BGX_D bool substep_impl(const float* __restrict__ M, float* q, float* qd,
         tape[TL::RS + o + TL::NRC + i] = lv.at(3, i);
       }
     }
-    // line search: trial x+ = relu(y - eta g), residual into r
+    // line search: trial x+ = relu(y - eta g), tested as f(x+) - f(y) >
+    // g.d + |d|^2 / (2 eta), d = x+ - y, the residual into r.  A topology that
+    // a lane-per-leg kernel steps tests it as that kernel does (bgx_star.h):
+    // |A d|^2 / 2 > |d|^2 / (2 eta), A d into r, equal in exact arithmetic.  At
+    // a tie the two round apart, and the tape is to take the steps that made
+    // the states.
+    constexpr bool BY_AD = star_ok<T>();
     bool cond = true;
     for (int ls = 0; ls <= maxls && cond; ++ls) {
       if (ls > 0) eta *= 0.5f;
       const float e_ = eta;
+      if constexpr (BY_AD) {
+        float ad = 0.f, dd = 0.f;
+        auto d_slot = [&](int s, int k) {
+          return fmaxf(rows.at(RV_Y, s, k) - e_ * rows.at(RV_G, s, k), 0.f) - rows.at(RV_Y, s, k);
+        };
+        auto d_lim = [&](int i) {
+          return fmaxf(lv.at(1, i) - e_ * lv.at(2, i), 0.f) - lv.at(1, i);
+        };
+        apply_a(d_slot, d_lim,
+                [&](int s, int k, float o) {
+                  rows.at(RV_R, s, k) = o;
+                  ad += o * o;
+                  const float df = d_slot(s, k);
+                  dd += df * df;
+                },
+                [&](int i, float o) {
+                  lv.at(3, i) = o;
+                  ad += o * o;
+                  const float df = d_lim(i);
+                  dd += df * df;
+                },
+                no_z);
+        trials += 1;
+        cond = e_ * (0.5f * ad) > 0.5f * dd + lseps;
+        continue;
+      }
       float fx = 0.f, dg = 0.f, dd = 0.f;
       apply_a([&](int s, int k) {
                 return fmaxf(rows.at(RV_Y, s, k) - e_ * rows.at(RV_G, s, k), 0.f);
@@ -1424,17 +1457,20 @@ BGX_D bool substep_impl(const float* __restrict__ M, float* q, float* qd,
       trials += 1;
       cond = e_ * (fx - fy) > e_ * dg + 0.5f * dd + lseps;
     }
-    // error at x+: |relu(x+ - grad f(x+)) - x+| with grad = A^T (A x+ + b)
+    // error at x+: |relu(x+ - grad f(x+)) - x+|, grad f(x+) = A^T (A x+ + b),
+    // which is g + A^T A d
     float e2 = 0.f;
     const float e_ = eta;
     apply_a([&](int s, int k) { return rows.at(RV_R, s, k); },
             [&](int i) { return lv.at(3, i); },
             [&](int s, int k, float o) {
+              if constexpr (BY_AD) o = rows.at(RV_G, s, k) + o;
               const float xp = fmaxf(rows.at(RV_Y, s, k) - e_ * rows.at(RV_G, s, k), 0.f);
               const float dv = fmaxf(xp - o, 0.f) - xp;
               e2 += dv * dv;
             },
             [&](int i, float o) {
+              if constexpr (BY_AD) o = lv.at(2, i) + o;
               const float xp = fmaxf(lv.at(1, i) - e_ * lv.at(2, i), 0.f);
               const float dv = fmaxf(xp - o, 0.f) - xp;
               e2 += dv * dv;

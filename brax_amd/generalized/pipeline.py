@@ -271,8 +271,9 @@ def pipeline_step(sys: S.System, state: State, act, n_frames: int = 1,
 
   Differentiable like the reference's step under jax.grad: when q, qd or
   act require gradients, the new q and qd carry them through the
-  hand-written adjoint (a one-step ``rollout_grad``), and the frames x, xd
-  of the returned State carry them on to q and qd (``frames``).  With
+  hand-written adjoint (that of a one-step ``rollout_grad``; the values are
+  those of a step without gradients), and the frames x, xd of the returned
+  State carry them on to q and qd (``frames``).  With
   debug=True the State carries the contacts of the new state
   (``contacts``).
   """
@@ -284,7 +285,8 @@ def pipeline_step(sys: S.System, state: State, act, n_frames: int = 1,
       a = (a[None] if a.dim() == 1 else a).expand(n, m.nu)[None]
     else:
       a = torch.zeros(1, n, 0, device=m.device)
-    qt, qdt, status = rollout_grad(sys, state.q, state.qd, a, n_frames, ckpt_every=1)
+    qt, qdt, status = _rollout_grad(sys, state.q, state.qd, a, n_frames, 1, False,
+                                    "bgx_rollout_from")
     q, qd = qt[0], qdt[0]
     x, xd = frames(sys, q, qd)
     return _with_contacts(sys, State(q=q, qd=qd, x=x, xd=xd, status=status), debug)
@@ -369,24 +371,23 @@ def probe(sys: S.System, state: State, act, n_frames: int = 1) -> Dict[str, torc
 
 
 class _RolloutFn(torch.autograd.Function):
-  """Differentiable rollout: forward = bgx_rollout with the trajectory,
-  backward = bgx_rollout_adjoint (segments of ckpt_every env steps are
-  recomputed from their checkpoints)."""
+  """Differentiable rollout: forward = ``fn`` (bgx_rollout_primal, or
+  bgx_rollout_from) with the trajectory, backward = bgx_rollout_adjoint
+  (segments of ckpt_every env steps are recomputed from their checkpoints)."""
 
   @staticmethod
-  def forward(ctx, q0, qd0, acts, m, n_frames, ckpt_every, min_workspace):
+  def forward(ctx, q0, qd0, acts, m, n_frames, ckpt_every, min_workspace, fn):
     n, T = q0.shape[0], acts.shape[0]
     q_in, qd_in, q, qd = _state_io(q0.detach(), qd0.detach())
     a = acts.detach().contiguous()
     qt = torch.empty(T, n, m.nq, device=m.device)
     qdt = torch.empty(T, n, m.nv, device=m.device)
     status = torch.empty(n, dtype=torch.int32, device=m.device)
-    lib = _lib.load()
-    _lib.check(lib.bgx_rollout_from(m.handle, n, T, int(n_frames), _lib.ptr(q_in),
-                                    _lib.ptr(qd_in), _lib.ptr(q), _lib.ptr(qd),
-                                    _lib.ptr(a) if m.nu else None, n * m.nu, _lib.ptr(qt),
-                                    _lib.ptr(qdt), None, None, None, None, _lib.ptr(status),
-                                    _stream()))
+    step = getattr(_lib.load(), fn)
+    _lib.check(step(m.handle, n, T, int(n_frames), _lib.ptr(q_in), _lib.ptr(qd_in),
+                    _lib.ptr(q), _lib.ptr(qd), _lib.ptr(a) if m.nu else None, n * m.nu,
+                    _lib.ptr(qt), _lib.ptr(qdt), None, None, None, None, _lib.ptr(status),
+                    _stream()))
     idx = list(range(ckpt_every - 1, T - 1, ckpt_every))
     ckq = torch.cat([q0.detach()[None].contiguous(), qt[idx]], 0).contiguous()
     ckqd = torch.cat([qd0.detach()[None].contiguous(), qdt[idx]], 0).contiguous()
@@ -419,7 +420,7 @@ class _RolloutFn(torch.autograd.Function):
         _lib.ptr(a) if m.nu else None, n * m.nu, _lib.ptr(gqt), _lib.ptr(gqdt),
         _lib.ptr(gact) if m.nu else None, _lib.ptr(gq0), _lib.ptr(gqd0), _lib.ptr(ws),
         nbytes, _lib.ptr(status), _stream()))
-    return gq0, gqd0, gact, None, None, None, None
+    return gq0, gqd0, gact, None, None, None, None, None
 
 
 def rollout_grad(sys: S.System, q0: torch.Tensor, qd0: torch.Tensor, acts: torch.Tensor,
@@ -432,8 +433,15 @@ def rollout_grad(sys: S.System, q0: torch.Tensor, qd0: torch.Tensor, acts: torch
   pipeline.step, brax/training/agents/apg/train.py:188-198).  The backward
   pass recomputes segments of ``ckpt_every`` env steps from checkpoints.
   With ``min_workspace`` the backward pass takes the least workspace (one
-  substep's tape at a time) instead of a whole segment's tapes.
+  substep's tape at a time) instead of a whole segment's tapes.  The states
+  are those that the backward pass repeats (bgx_rollout_primal); ``rollout``'s
+  agree with them within rounding.
   """
+  return _rollout_grad(sys, q0, qd0, acts, n_frames, ckpt_every, min_workspace,
+                       "bgx_rollout_primal")
+
+
+def _rollout_grad(sys, q0, qd0, acts, n_frames, ckpt_every, min_workspace, fn):
   m = device_model(sys, q0.device)
   if q0.dim() != 2 or q0.shape[1] != m.nq or qd0.shape != (q0.shape[0], m.nv):
     raise ValueError("q0 must be (N, q_size) and qd0 (N, qd_size)")
@@ -442,4 +450,4 @@ def rollout_grad(sys: S.System, q0: torch.Tensor, qd0: torch.Tensor, acts: torch
   if ckpt_every < 1 or n_frames < 1:
     raise ValueError("ckpt_every and n_frames must be positive")
   return _RolloutFn.apply(q0.float(), qd0.float(), acts.float(), m, n_frames, ckpt_every,
-                          min_workspace)
+                          min_workspace, fn)

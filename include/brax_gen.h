@@ -153,6 +153,17 @@ int bgx_rollout_from(const bgx_model* model, int32_t n_envs, int32_t n_steps,
                      float* qd_traj, float* x_pos, float* x_rot, float* xd_ang,
                      float* xd_vel, int32_t* status, void* stream);
 
+/* bgx_rollout_from on the kernel that bgx_rollout_adjoint recomputes segments
+ * with: the forward pass whose states the adjoint repeats bit for bit.  It is
+ * bgx_rollout_from itself but for four-legged topologies, which it steps at
+ * one thread per env whatever BGX_KERNELS_LANES says (the states agree within
+ * rounding). */
+int bgx_rollout_primal(const bgx_model* model, int32_t n_envs, int32_t n_steps,
+                       int32_t n_frames, const float* q_in, const float* qd_in, float* q,
+                       float* qd, const float* act, int64_t act_step_stride, float* q_traj,
+                       float* qd_traj, float* x_pos, float* x_rot, float* xd_ang,
+                       float* xd_vel, int32_t* status, void* stream);
+
 /* bgx_init, with copies of q_in and qd_in into q and qd. */
 int bgx_init_copy(const bgx_model* model, int32_t n_envs, const float* q_in,
                   const float* qd_in, float* q, float* qd, float* x_pos, float* x_rot,
