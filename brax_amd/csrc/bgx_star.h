@@ -294,16 +294,37 @@ struct StarRows {
       for (int k = 0; k < W; ++k) r[i][x][k] = v[k];
     }
   }
-  BGX_D void get(int i, int x, float* v) const {
-    if constexpr (LDS) {
+  BGX_D void get(int i, float (*v)[W]) const {
 #pragma unroll
-      for (int q = 0; q < Q; ++q) {
-        const float4 f = base[((i * 3 + x) * Q + q) * WAVE];
-        v[4 * q] = f.x, v[4 * q + 1] = f.y, v[4 * q + 2] = f.z, v[4 * q + 3] = f.w;
+    for (int x = 0; x < 3; ++x) {
+      if constexpr (LDS) {
+#pragma unroll
+        for (int q = 0; q < Q; ++q) {
+          const float4 f = base[((i * 3 + x) * Q + q) * WAVE];
+          v[x][4 * q] = f.x, v[x][4 * q + 1] = f.y, v[x][4 * q + 2] = f.z, v[x][4 * q + 3] = f.w;
+        }
+      } else {
+#pragma unroll
+        for (int k = 0; k < W; ++k) v[x][k] = r[i][x][k];
       }
-    } else {
+    }
+  }
+  // fn(i, rows of slot i) for the slots that are on.  The next slot's rows are
+  // read before, on or not (an unused slot's are never looked at): behind its
+  // branch, they would be waited for with nothing else to do.
+  template <class Fn>
+  BGX_D void each(const bool* on, Fn fn) const {
+    float next[3][W];
+    if (Star<T>::S > 0) get(0, next);
 #pragma unroll
-      for (int k = 0; k < W; ++k) v[k] = r[i][x][k];
+    for (int i = 0; i < Star<T>::S; ++i) {
+      float j[3][W];
+#pragma unroll
+      for (int x = 0; x < 3; ++x)
+#pragma unroll
+        for (int k = 0; k < W; ++k) j[x][k] = next[x][k];
+      if (i + 1 < Star<T>::S) get(i + 1, next);
+      if (on[i]) fn(i, j);
     }
   }
 };
@@ -672,67 +693,78 @@ BGX_D int star_substep(float* ml, int b, StarState<T>& s, const float* act,
       for (int k = 0; k < 4; ++k) X[i][k] = Y[i][k] = G[i][k] = R[i][k] = 0.f;
 #pragma unroll
     for (int k = 0; k < K; ++k) xl[k] = yl[k] = gl[k] = rl[k] = 0.f;
-    // t = (L^-T J^T) in
-    auto gather = [&](auto in, auto in_l, float* t, float* tr) {
-      float p[6] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+    // products with A = P^T P + diag, P = L^-T J^T.  A sweep over the rows ends
+    // one product and begins the next, t being P in of the product that ends:
+    // out receives A in, then nxt gives the next input of the same row, summed
+    // into t.  So a product reads its rows once, where summing and applying in
+    // turn reads them twice, and where rows live in LDS those reads (1 KB an
+    // instruction) are the solver's longest stretch.  65,536 quadrupeds, us a
+    // substep, the same bits: 130 -> 94 over 40 env steps from a standing
+    // start, 166 -> 117 once settled on the floor.
+    float t[K], tr[6], p[6];
+    auto add_slot = [&](int i, const float (*j)[SRows::W], auto nxt) {
+      const float v0 = nxt(i, 0), v1 = nxt(i, 1), v2 = nxt(i, 2), v3_ = nxt(i, 3);
+      const float a[3] = {(v0 + v1) + (v2 + v3_), v0 - v1, v2 - v3_};
+#pragma unroll
+      for (int x = 0; x < 3; ++x) {
+#pragma unroll
+        for (int k = 0; k < K; ++k)
+          if (k <= SR::link(i)) t[k] += a[x] * j[x][k];
+#pragma unroll
+        for (int k = 0; k < 6; ++k) p[k] += a[x] * j[x][K + k];
+      }
+    };
+    auto add_limit = [&](int k, float v) {
+#pragma unroll
+      for (int j = 0; j <= k; ++j) t[j] += v * ll[k][j];
+#pragma unroll
+      for (int j = 0; j < 6; ++j) p[j] += v * lr[k][j];
+    };
+    auto clear = [&]() {
 #pragma unroll
       for (int k = 0; k < K; ++k) t[k] = 0.f;
 #pragma unroll
-      for (int i = 0; i < S; ++i) {
-        if (on[i]) {
-          const float v0 = in(i, 0), v1 = in(i, 1), v2 = in(i, 2), v3_ = in(i, 3);
-          const float a[3] = {(v0 + v1) + (v2 + v3_), v0 - v1, v2 - v3_};
-#pragma unroll
-          for (int x = 0; x < 3; ++x) {
-            float j[SRows::W];
-            J.get(i, x, j);
-#pragma unroll
-            for (int k = 0; k < K; ++k)
-              if (k <= SR::link(i)) t[k] += a[x] * j[k];
-#pragma unroll
-            for (int k = 0; k < 6; ++k) p[k] += a[x] * j[K + k];
-          }
-        }
-      }
-      if (on_l) {
-#pragma unroll
-        for (int k = 0; k < K; ++k) {
-          if (!star_lim<T>(6 + k)) continue;
-          const float v = in_l(k);
-#pragma unroll
-          for (int j = 0; j <= k; ++j) t[j] += v * ll[k][j];
-#pragma unroll
-          for (int j = 0; j < 6; ++j) p[j] += v * lr[k][j];
-        }
-      }
+      for (int k = 0; k < 6; ++k) p[k] = 0.f;
+    };
+    auto sum_root = [&]() {
 #pragma unroll
       for (int k = 0; k < 6; ++k) tr[k] = quad_sum(p[k]);
     };
-    // out = A in
-    auto apply = [&](auto in, auto in_l, auto out, auto out_l) {
-      float t[K], tr[6];
-      gather(in, in_l, t, tr);
+    // t = P nxt
+    auto gather = [&](auto nxt, auto nxt_l) {
+      clear();
+      J.each(on, [&](int i, const float (*j)[SRows::W]) { add_slot(i, j, nxt); });
+      if (on_l) {
 #pragma unroll
-      for (int i = 0; i < S; ++i) {
-        if (on[i]) {
-          float e[3];
-#pragma unroll
-          for (int x = 0; x < 3; ++x) {
-            float j[SRows::W];
-            J.get(i, x, j);
-            e[x] = 0.f;
-#pragma unroll
-            for (int k = 0; k < 6; ++k) e[x] += j[K + k] * tr[k];
-#pragma unroll
-            for (int k = 0; k < K; ++k)
-              if (k <= SR::link(i)) e[x] += j[k] * t[k];
-          }
-          out(i, 0, e[0] + e[1] + diag[i] * in(i, 0));
-          out(i, 1, e[0] - e[1] + diag[i] * in(i, 1));
-          out(i, 2, e[0] + e[2] + diag[i] * in(i, 2));
-          out(i, 3, e[0] - e[2] + diag[i] * in(i, 3));
-        }
+        for (int k = 0; k < K; ++k)
+          if (star_lim<T>(6 + k)) add_limit(k, nxt_l(k));
       }
+      sum_root();
+    };
+    // out = A in (t = P in), then t = P nxt where next says so
+    auto sweep = [&](auto in, auto in_l, auto out, auto out_l, auto next, auto nxt, auto nxt_l) {
+      constexpr bool NEXT = decltype(next)::value;
+      float u_[K];
+#pragma unroll
+      for (int k = 0; k < K; ++k) u_[k] = t[k];
+      if constexpr (NEXT) clear();
+      J.each(on, [&](int i, const float (*j)[SRows::W]) {
+        float e[3];
+#pragma unroll
+        for (int x = 0; x < 3; ++x) {
+          e[x] = 0.f;
+#pragma unroll
+          for (int k = 0; k < 6; ++k) e[x] += j[x][K + k] * tr[k];
+#pragma unroll
+          for (int k = 0; k < K; ++k)
+            if (k <= SR::link(i)) e[x] += j[x][k] * u_[k];
+        }
+        out(i, 0, e[0] + e[1] + diag[i] * in(i, 0));
+        out(i, 1, e[0] - e[1] + diag[i] * in(i, 1));
+        out(i, 2, e[0] + e[2] + diag[i] * in(i, 2));
+        out(i, 3, e[0] - e[2] + diag[i] * in(i, 3));
+        if constexpr (NEXT) add_slot(i, j, nxt);
+      });
       if (on_l) {
 #pragma unroll
         for (int k = 0; k < K; ++k) {
@@ -741,90 +773,114 @@ BGX_D int star_substep(float* ml, int b, StarState<T>& s, const float* act,
 #pragma unroll
           for (int j = 0; j < 6; ++j) e += lr[k][j] * tr[j];
 #pragma unroll
-          for (int j = 0; j <= k; ++j) e += ll[k][j] * t[j];
+          for (int j = 0; j <= k; ++j) e += ll[k][j] * u_[j];
           out_l(k, e + ldiag[k] * in_l(k));
+          if constexpr (NEXT) add_limit(k, nxt_l(k));
         }
       }
+      if constexpr (NEXT) sum_root();
     };
+    // A product that may not be wanted (after a rejected or a last step) begins
+    // in the sweep before it only where that saves reads of LDS.  Ants, whose
+    // rows are in registers, take 18.4 us a substep at 4,096 without and 20.6
+    // with it.
+    constexpr std::true_type always{};
+    constexpr std::bool_constant<SRows::LDS> if_lds{};
     const int maxiter = (int)ml[H_MAXITER], maxls = (int)ml[H_MAXLS];
     const float tol = ml[H_TOL], lseps = ml[H_LSEPS];
-    float tk = 1.f, eta = 1.f, err = INFINITY;
-    bool running = has_rows;
-    for (int it = 0; it < maxiter; ++it) {
-      if (it > 0) running = running && (err > tol);
-      if (!running) break;
-      // gradient at y: r = A y + b, g = A^T r
-      apply([&](int i, int k) { return Y[i][k]; }, [&](int k) { return yl[k]; },
-            [&](int i, int k, float o) { R[i][k] = o + sb[i][k]; },
-            [&](int k, float o) { rl[k] = o + lb[k]; });
-      apply([&](int i, int k) { return R[i][k]; }, [&](int k) { return rl[k]; },
-            [&](int i, int k, float o) { G[i][k] = o; }, [&](int k, float o) { gl[k] = o; });
+    float tk = 1.f, eta = 1.f, err;
+    auto y_ = [&](int i, int k) { return Y[i][k]; };
+    auto y_l = [&](int k) { return yl[k]; };
+    auto r_ = [&](int i, int k) { return R[i][k]; };
+    auto r_l = [&](int k) { return rl[k]; };
+    // x+ = relu(y - eta g) and d = x+ - y
+    auto x_ = [&](int i, int k) { return fmaxf(Y[i][k] - eta * G[i][k], 0.f); };
+    auto x_l = [&](int k) { return fmaxf(yl[k] - eta * gl[k], 0.f); };
+    auto d_ = [&](int i, int k) { return x_(i, k) - Y[i][k]; };
+    auto d_l = [&](int k) { return x_l(k) - yl[k]; };
+    // the residual at y = 0
+#pragma unroll
+    for (int i = 0; i < S; ++i)
+#pragma unroll
+      for (int k = 0; k < 4; ++k) R[i][k] = sb[i][k];
+#pragma unroll
+    for (int k = 0; k < K; ++k) rl[k] = lb[k];
+    bool running = has_rows && maxiter > 0;
+    if (running) gather(r_, r_l);
+    for (int it = 0; running; ++it) {
+      // R is the residual r = A y + b: the gradient at y is g = A^T r
+      float dd = 0.f;
+      auto next_d = [&](int i, int k) {
+        const float d = d_(i, k);
+        dd += d * d;
+        return d;
+      };
+      auto next_dl = [&](int k) {
+        const float d = d_l(k);
+        dd += d * d;
+        return d;
+      };
+      sweep(r_, r_l, [&](int i, int k, float o) { G[i][k] = o; },
+            [&](int k, float o) { gl[k] = o; }, always, next_d, next_dl);
       // line search over x+ = relu(y - eta g).  f is quadratic, so with
       // d = x+ - y its test f(x+) - f(y) > g.d + |d|^2 / (2 eta) is
       // |A d|^2 / 2 > |d|^2 / (2 eta), without the difference of two nearly
       // equal sums: fewer steps are decided by rounding (a tie still is), and
-      // the taped substep decides by the same test (bgx_step.h).  R holds A d.
-      bool cond = true;
-      for (int ls = 0; ls <= maxls && cond; ++ls) {
-        if (ls > 0) eta *= 0.5f;
-        const float e_ = eta;
-        float ad = 0.f, dd = 0.f;
-        apply([&](int i, int k) { return fmaxf(Y[i][k] - e_ * G[i][k], 0.f) - Y[i][k]; },
-              [&](int k) { return fmaxf(yl[k] - e_ * gl[k], 0.f) - yl[k]; },
+      // the taped substep decides by the same test (bgx_step.h).  R becomes
+      // A d, the next input if the step is taken.
+      for (int ls = 0;; ++ls) {
+        float ad = 0.f;
+        sweep(d_, d_l,
               [&](int i, int k, float o) {
                 R[i][k] = o;
                 ad += o * o;
-                const float d = fmaxf(Y[i][k] - e_ * G[i][k], 0.f) - Y[i][k];
-                dd += d * d;
               },
               [&](int k, float o) {
                 rl[k] = o;
                 ad += o * o;
-                const float d = fmaxf(yl[k] - e_ * gl[k], 0.f) - yl[k];
-                dd += d * d;
-              });
-        ad = quad_sum(ad), dd = quad_sum(dd);
+              },
+              if_lds, r_, r_l);
         trials += 1;
-        cond = e_ * (0.5f * ad) > 0.5f * dd + lseps;
+        if (!(eta * (0.5f * quad_sum(ad)) > 0.5f * quad_sum(dd) + lseps) || ls >= maxls) break;
+        eta *= 0.5f;
+        dd = 0.f;
+        gather(next_d, next_dl);
       }
-      // error at x+: |relu(x+ - grad f(x+)) - x+|, grad f(x+) = g + A^T A d
-      const float e_ = eta;
-      float e2 = 0.f;
-      apply([&](int i, int k) { return R[i][k]; }, [&](int k) { return rl[k]; },
-            [&](int i, int k, float o) {
-              const float xn = fmaxf(Y[i][k] - e_ * G[i][k], 0.f);
-              const float dv = fmaxf(xn - (G[i][k] + o), 0.f) - xn;
-              e2 += dv * dv;
-            },
-            [&](int k, float o) {
-              const float xn = fmaxf(yl[k] - e_ * gl[k], 0.f);
-              const float dv = fmaxf(xn - (gl[k] + o), 0.f) - xn;
-              e2 += dv * dv;
-            });
-      err = fsqrt(quad_sum(e2));
+      if constexpr (!if_lds) gather(r_, r_l);
+      // error at x+: |relu(x+ - grad f(x+)) - x+|, grad f(x+) = g + A^T A d;
+      // and the next y, x+ + beta (x+ - x)
       const float tn = 0.5f * (1.f + fsqrt(1.f + 4.f * tk * tk));
       const float beta = (tk - 1.f) * rcp(tn);
-#pragma unroll
-      for (int i = 0; i < S; ++i)
-#pragma unroll
-        for (int k = 0; k < 4; ++k) {
-          const float xn = fmaxf(Y[i][k] - e_ * G[i][k], 0.f);
-          Y[i][k] = xn + beta * (xn - X[i][k]);
-          X[i][k] = xn;
-        }
-#pragma unroll
-      for (int k = 0; k < K; ++k) {
-        const float xn = fmaxf(yl[k] - e_ * gl[k], 0.f);
-        yl[k] = xn + beta * (xn - xl[k]);
-        xl[k] = xn;
-      }
+      float e2 = 0.f;
+      sweep(r_, r_l,
+            [&](int i, int k, float o) {
+              const float xn = x_(i, k);
+              const float dv = fmaxf(xn - (G[i][k] + o), 0.f) - xn;
+              e2 += dv * dv;
+              Y[i][k] = xn + beta * (xn - X[i][k]);
+              X[i][k] = xn;
+            },
+            [&](int k, float o) {
+              const float xn = x_l(k);
+              const float dv = fmaxf(xn - (gl[k] + o), 0.f) - xn;
+              e2 += dv * dv;
+              yl[k] = xn + beta * (xn - xl[k]);
+              xl[k] = xn;
+            },
+            if_lds, y_, y_l);
+      err = fsqrt(quad_sum(e2));
       eta = eta <= 1e-6f ? 1.f : eta * 2.f;
       tk = tn;
       iters += 1;
+      running = err > tol && it + 1 < maxiter;
+      if (running) {
+        if constexpr (!if_lds) gather(y_, y_l);
+        sweep(y_, y_l, [&](int i, int k, float o) { R[i][k] = o + sb[i][k]; },
+              [&](int k, float o) { rl[k] = o + lb[k]; }, always, r_, r_l);
+      }
     }
     // ---- qdd = u + L^-1 (L^-T J^T) x (integrator.py:58-64)
-    float t[K], tr[6];
-    gather([&](int i, int k) { return X[i][k]; }, [&](int k) { return xl[k]; }, t, tr);
+    gather([&](int i, int k) { return X[i][k]; }, [&](int k) { return xl[k]; });
     F.l(t, tr);
 #pragma unroll
     for (int k = 0; k < K; ++k) u[k] = has_rows ? u[k] + t[k] : u[k];
@@ -904,14 +960,26 @@ BGX_D void star_stage(const float* M, float* lds) {
   __syncthreads();
 }
 
+// The LDS of a wavefront in star_item: one object for every kernel that calls
+// it, so that its address is a constant there.  Behind a pointer from two
+// callers the same substep took 512 registers and 640 bytes of scratch a lane
+// instead of 378 and 400 (65,536 quadrupeds, one substep with its frames: 147
+// us instead of 109).
+template <class T>
+BGX_D float* star_smem() {
+  constexpr int N = star_lds_floats<T>();
+  __shared__ __align__(16) float mem[T::BATCH && CHAIN_LDS_FLOATS > N ? CHAIN_LDS_FLOATS : N];
+  return mem;
+}
+
 // The envs of one item (up to STAR_ENVS), n_steps x n_frames substeps.  An
 // env past the item's count computes on the item's last env and writes
 // nothing.  A function of its own (as chain_item): the homogeneous kernel and
 // the batch kernel call the same code.
 template <class T>
-BGX_ITEM void star_item(const Launch& a, const BatchItem& it, float* lds_) {
+BGX_ITEM void star_item(const Launch& a, const BatchItem& it) {
   constexpr int K = Star<T>::K, NQ = T::NQ, NV = T::NV, NU = T::NU;
-  float* lds = star_lds(lds_);
+  float* lds = star_smem<T>();
   const int b = threadIdx.x % STAR_LEGS, e = threadIdx.x / STAR_LEGS;
   const bool live = e < it.n;
   const int ec = live ? e : it.n - 1;
@@ -986,21 +1054,18 @@ BGX_D BatchItem star_home_item(const Launch& a) {
 
 template <class T>
 __global__ __launch_bounds__(WAVE) void k_star(Launch a) {
-  __shared__ __align__(16) float lds[star_lds_floats<T>()];
-  star_item<T>(a, star_home_item<T>(a), lds);
+  star_item<T>(a, star_home_item<T>(a));
 }
 
 // the batch kernel (bgx_batch.h) of a topology of this shape
 template <class T>
 __global__ __launch_bounds__(WAVE) void k_star_batch(Launch a) {
-  constexpr int N = star_lds_floats<T>();
-  __shared__ __align__(16) float smem[N > CHAIN_LDS_FLOATS ? N : CHAIN_LDS_FLOATS];
   for (;;) {
     const int i = next_item(a);
     if (i < 0) break;
     const BatchItem it = a.items[i];
-    if (it.kind == BATCH_CHAIN) run_chain_item(a, it, smem);
-    else star_item<T>(a, it, smem);
+    if (it.kind == BATCH_CHAIN) run_chain_item(a, it, star_smem<T>());
+    else star_item<T>(a, it);
     __syncthreads();  // the next item reuses the LDS
   }
   batch_done(a);
