@@ -186,31 +186,25 @@ int bgx_model_set_launch(bgx_model* m, int kernels, int32_t envs_per_workgroup) 
   return BGX_OK;
 }
 
+// Lanes per env of the step kernels.  By the settings alone, never by the
+// batch: an env's result does not depend on the envs or the steps around it.
+// A lane per leg is the default at every size.  Against one thread per env, us
+// a substep of quadrupeds settled on the floor: 32,768 in env steps of their
+// own 74 / 122-200, 65,536 111-142 / 175-305 and over 1,000 env steps in one
+// launch 117 / 114, 131,072 226 / 224; of ants 65,536 60 / 142.
+static int step_lanes(const bgx_model* m) {
+  const int w = kOps[m->topo]->mlanes;
+  if (m->lanes) return m->lanes;
+  if (w == bgx::STAR_LEGS && m->kc) return 1;  // the tile is the one-thread kernel's
+  return w ? w : 1;
+}
+
 int bgx_model_get_launch(const bgx_model* m, int kernels) {
   if (m && kernels == BGX_KERNELS_TILE) return m->kc ? m->kc : kOps[m->topo]->tiles[0];
-  if (m && kernels == BGX_KERNELS_LANES) {
-    const int w = kOps[m->topo]->mlanes;
-    return m->lanes ? m->lanes : (w ? w : 1);
-  }
+  if (m && kernels == BGX_KERNELS_LANES) return step_lanes(m);
   if (m && kernels == BGX_KERNELS_ADJOINT_PARTS) return m->adj_parts;
   if (!m || (kernels != BGX_KERNELS_STEP && kernels != BGX_KERNELS_ADJOINT)) return -1;
   return m->epw[kernels] ? m->epw[kernels] : bgx::WAVE;
-}
-
-// Lanes per env of a rollout of n envs over n_sub substeps (Launch::lanes).
-// A lane per leg needs four wavefronts for 64 envs, each alone on its SIMD:
-// up to two for every SIMD (32,768 envs) it is faster at any contact load
-// (quadrupeds settled on the floor: 86 us a substep against 114 with one
-// thread per env).  At 65,536 it is as fast over the first substeps from a
-// standing start (141 us against 146), but long rollouts settle, the solver
-// grows, and one thread per env takes over: 171 us a substep against 110 over
-// 1,000 env steps.
-static int rollout_lanes(const bgx_model* m, int64_t n, int64_t n_sub) {
-  constexpr int64_t kStarEnvs = 2 * 16 * 1024, kStarSubsteps = 25;
-  if (m->lanes == 0 && kOps[m->topo]->mlanes == bgx::STAR_LEGS && n > kStarEnvs &&
-      n_sub > kStarSubsteps)
-    return 1;
-  return m->lanes;
 }
 
 // Lanes per env of the states that the adjoint differentiates, forward and
@@ -218,7 +212,7 @@ static int rollout_lanes(const bgx_model* m, int64_t n, int64_t n_sub) {
 // the code that stage A1 tapes (bgx_step.h), so that the tape starts from and
 // arrives at the same bits.
 static int primal_lanes(const bgx_model* m) {
-  return kOps[m->topo]->mlanes == bgx::STAR_LEGS ? 1 : m->lanes;
+  return kOps[m->topo]->mlanes == bgx::STAR_LEGS ? 1 : step_lanes(m);
 }
 
 enum class Run { INIT, STEP, PRIMAL };
@@ -235,8 +229,7 @@ static int launch(const bgx_model* m, Run run, bgx::Launch a, void* stream) {
   a.M = m->table;
   a.epw = m->epw[BGX_KERNELS_STEP];
   a.kc = m->kc;
-  a.lanes = run == Run::PRIMAL ? primal_lanes(m)
-                               : rollout_lanes(m, a.n, (int64_t)a.n_steps * a.n_frames);
+  a.lanes = run == Run::PRIMAL ? primal_lanes(m) : step_lanes(m);
   const bgx::TopoOps* ops = kOps[m->topo];
   a.q_step = (long long)a.n * ops->dims[1], a.qd_step = (long long)a.n * ops->dims[2];
   if ((a.q_traj || a.qd_traj) && a.n_seg > 1)

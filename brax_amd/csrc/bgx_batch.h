@@ -19,8 +19,8 @@
 // (k_rollout<NoTree, true> for chains), forming one item per workgroup from
 // blockIdx.  Both reach an env's substeps through the same function
 // (star_item, chain_item) or the one call site (tree_item), so an env's arithmetic is the same compiled code whether it runs alone, in
-// a batch of its kind, or in a mixed batch: results are bitwise equal (the
-// GPU tests compare them).
+// a batch of its kind, or in a mixed batch: results are bitwise equal at the
+// models' default launch settings (the GPU tests compare them).
 #pragma once
 
 #include <hip/hip_runtime.h>

@@ -586,9 +586,7 @@ struct Ops {
       }
     }
     if constexpr (star_ok<T>()) {
-      // a lane per leg, unless the caller chose one thread per env or one of
-      // that kernel's slot counts
-      if (a.lanes != 1 && a.kc == 0) {
+      if (a.lanes != 1) {
         const dim3 g = env_grid(a.n, STAR_ENVS);
         hipLaunchKernelGGL(k_star<T>, dim3(g.x, a.n_seg > 1 ? (unsigned)a.n_seg : 1u),
                            dim3(WAVE), 0, s, a);

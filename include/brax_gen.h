@@ -97,10 +97,11 @@ int bgx_model_topology(const bgx_model* model);
  * one thread per env; the topology's multi-lane width (the default, 0,
  * where the topology is compiled with a multi-lane kernel) runs an env on a
  * group of lanes: 4 for a free root with four equal legs (a lane per leg),
- * a lane per dof for other large trees.  The two agree within rounding; the
- * getter returns the width.  A four-legged topology runs at one thread per
- * env all the same where an LDS tile is chosen, and in rollouts of more than
- * 32,768 envs over more than 25 substeps. */
+ * a lane per dof for other large trees.  The two agree within rounding.  With
+ * 0, a four-legged topology runs one thread per env where an LDS tile is
+ * chosen (BGX_KERNELS_TILE; the multi-lane kernels have none).  The getter
+ * returns the lanes per env in use.  They never depend on the batch or the
+ * step count: an env's result is the same bits in any batch of its model. */
 #define BGX_KERNELS_LANES 3
 /* kernels = BGX_KERNELS_ADJOINT_PARTS splits bgx_rollout_adjoint's backward
  * pass into that many parts of whole envs (1-4; 0 = one), each on its own
@@ -256,7 +257,9 @@ int bgx_batch_sizes(const bgx_batch* batch, int64_t* sizes);
  * applies act + t * act_step_stride (packed, NULL = zero action);
  * q_traj (n_steps, q floats) and qd_traj receive the state after every env
  * step when non-NULL; status (envs) the BGX_STATUS_NONFINITE bit per env.
- * Each env's results are bitwise those of bgx_rollout on its model alone.
+ * Each env's results are bitwise those of bgx_rollout on its model alone at
+ * the default launch settings (the batch does not read BGX_KERNELS_LANES and
+ * BGX_KERNELS_TILE).
  * The batch's work counter is shared by its launches: launches of one batch
  * must not overlap (one stream).  Graph-capturable. */
 int bgx_batch_rollout(const bgx_batch* batch, int32_t n_steps, int32_t n_frames, float* q,
