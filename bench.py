@@ -184,25 +184,22 @@ def forward_bench(args, name):
   acts.uniform_(-act_range, act_range, generator=g)
   q_init = torch.tensor(q0, device=dev)
   qd_init = torch.tensor(qd0, device=dev)
-  epw, kc = 64, None
+  epw = 64
   from brax_amd.generalized import autotune
   if args.lanes:
     autotune.set_launch(m, autotune.LANES, args.lanes)
-  lanes = lib.bgx_model_get_launch(m.handle, 3)
-  kernel = {1: "k_rollout", 4: "k_star"}.get(lanes, "k_mtree")
-  if not args.no_tune:
-    # the tile trades occupancy against slow-path substeps, which grow as
-    # the envs settle onto the floor: time it over the timed steps (up to 20);
-    # 0: a multi-lane kernel was faster
-    kc = autotune.tune_tile(sys_, q_init, qd_init, acts[:min(K, 20)], N_FRAMES)
-    if lanes == 4 and kc:
-      lanes, kernel = 1, "k_rollout"
+  lanes = autotune.get_launch(m, autotune.LANES)
+  # the profile's kernel: k_mtree with its mass-matrix rows in registers
+  kernel = {1: "k_rollout", 4: "k_star"}.get(lanes, "k_mtree_rows")
   if lanes > 1:
     # a multi-lane kernel's workgroup is one wavefront of 64 / lanes envs,
     # and it keeps one contact row per candidate lane (no LDS tile)
-    epw, kc = 64 // lanes, None
+    epw = 64 // lanes
   elif not args.no_tune:
     epw = autotune.tune_step(sys_, q_init, qd_init, acts[:2], N_FRAMES)
+    # the tile trades occupancy against slow-path substeps, which grow as
+    # the envs settle onto the floor: time it over the timed steps (up to 20)
+    autotune.tune_tile(sys_, q_init, qd_init, acts[:min(K, 20)], N_FRAMES)
   q = q_init.clone()
   qd = qd_init.clone()
   status = torch.zeros(n, dtype=torch.int32, device=dev)
@@ -387,8 +384,7 @@ def fwd_adjoint_leg(n, T, ckpt, warmup, tune=True, cpu=True, parts=0):
   autotune.set_launch(m, autotune.ADJOINT_PARTS, parts)
   epw = [64, 64]
   if tune:
-    if autotune.get_launch(m, autotune.LANES) == 1:
-      epw[0] = autotune.tune_step(sys_, q0t, qd0t, acts0[:2], N_FRAMES)
+    epw[0] = autotune.tune_step(sys_, q0t, qd0t, acts0[:2], N_FRAMES)
     # the backward pass over one checkpoint segment: a shorter window times
     # the launch overheads rather than the kernels
     epw[1] = autotune.tune_adjoint(sys_, q0t, qd0t, acts0[:ckpt], N_FRAMES)

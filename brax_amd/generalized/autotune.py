@@ -8,13 +8,14 @@ of the 256 compute units with fewer lanes per workgroup.  Where the best
 point lies depends on the topology's registers and LDS per lane, so the
 tuner measures: it times a short rollout (or adjoint) per candidate on the
 model's own topology at the caller's batch size, keeps the fastest and
-remembers it per (topology, device, batch size, substeps).  The results of
-the kernels are bitwise the same for every launch shape; the choice is only
-about speed.  ``tune_tile`` picks the step kernels' LDS tile, the fast
-contact slots per env, among the compiled ones (results agree within
-rounding: an env with more active contacts than slots takes the
-slot-per-candidate path).  The reference has no counterpart (XLA picks its
-launch shapes).
+remembers it per (topology, device, batch size, substeps, horizon).  The
+results of the kernels are bitwise the same for every launch shape; the
+choice is only about speed.  ``tune_tile`` picks the one-thread kernel's LDS
+tile, the fast contact slots per env, among the compiled ones (results agree
+within rounding: an env with more active contacts than slots takes the
+slot-per-candidate path).  No tuner changes the lanes per env (LANES), which
+decide the kernel.  The reference has no counterpart (XLA picks its launch
+shapes).
 """
 
 from __future__ import annotations
@@ -63,8 +64,8 @@ def _time_ms(fn, reps: int) -> float:
   return best
 
 
-def _key(m, kernels, n, n_frames):
-  return (m.topo_id, str(m.device), kernels, n, n_frames)
+def _key(m, kernels, n, n_frames, horizon):
+  return (m.topo_id, str(m.device), kernels, n, n_frames, horizon, get_launch(m, LANES))
 
 
 def tiles(sys, device=None) -> Tuple[int, ...]:
@@ -76,9 +77,9 @@ def tiles(sys, device=None) -> Tuple[int, ...]:
   return tuple(int(buf[i]) for i in range(max(k, 0)))
 
 
-def _rollout_runner(m, q, qd, acts, n_frames):
-  """A callable running bgx_rollout over acts from copies of (q, qd)."""
-  lib = _lib.load()
+def _rollout_runner(m, q, qd, acts, n_frames, fn="bgx_rollout_from"):
+  """A callable running fn over acts from (q, qd)."""
+  step = getattr(_lib.load(), fn)
   n = q.shape[0]
   q0, qd0 = q.detach().float().contiguous(), qd.detach().float().contiguous()
   a = acts.detach().float().contiguous()
@@ -86,72 +87,62 @@ def _rollout_runner(m, q, qd, acts, n_frames):
   T = a.shape[0]
 
   def run():
-    qw.copy_(q0)
-    qdw.copy_(qd0)
-    _lib.check(lib.bgx_rollout(m.handle, n, T, int(n_frames), _lib.ptr(qw), _lib.ptr(qdw),
-                               _lib.ptr(a) if m.nu else None, n * m.nu, None, None, None,
-                               None, None, None, None, pipeline._stream()))
+    _lib.check(step(m.handle, n, T, int(n_frames), _lib.ptr(q0), _lib.ptr(qd0), _lib.ptr(qw),
+                    _lib.ptr(qdw), _lib.ptr(a) if m.nu else None, n * m.nu, None, None, None,
+                    None, None, None, None, pipeline._stream()))
   return run
+
+
+def _fastest(m, kernels, candidates, run, reps):
+  """The candidate setting with the least time, which is set on the model."""
+  times = {}
+  for c in candidates:
+    set_launch(m, kernels, c)
+    times[c] = _time_ms(run, reps)
+  best = min(times, key=times.get)
+  set_launch(m, kernels, best)
+  return best
 
 
 def tune_tile(sys, q: torch.Tensor, qd: torch.Tensor, acts: torch.Tensor, n_frames: int,
               reps: int = 3) -> int:
-  """Picks the step kernels' LDS tile (fast contact slots per env) for a
-  batch of q.shape[0] envs by timing bgx_rollout over acts with each
+  """Picks the one-thread step kernel's LDS tile (fast contact slots per env)
+  for a batch of q.shape[0] envs by timing a rollout over acts with each
   compiled tile.  More slots hold more envs' contacts on the fast path but
   take more LDS per env (fewer workgroups per compute unit); which wins
   depends on the batch's contact counts, which change as the envs settle,
   so acts should span the horizon of interest (a two-step window from
-  standing starts picks too few slots).  Where a lane per leg is the default,
-  that kernel is timed too: choice 0.  Returns the choice, which is
-  set on the model."""
+  standing starts picks too few slots).  Returns the choice, which is set on
+  the model.  A multi-lane kernel has no tile: a model that runs one is left
+  as it is (set LANES to 1 first)."""
   m = pipeline.device_model(sys, q.device)
-  n = q.shape[0]
-  key = _key(m, TILE, n, n_frames)
+  cands = tiles(sys, q.device)
+  if get_launch(m, LANES) > 1 or len(cands) <= 1:
+    return get_launch(m, TILE)
+  key = _key(m, TILE, q.shape[0], n_frames, acts.shape[0])
   if key in _CACHE:
     set_launch(m, TILE, _CACHE[key])
-    return _CACHE[key]
-  cands = tiles(sys, q.device)
-  if get_launch(m, LANES) == 4:
-    cands = (0,) + cands  # the lane-per-leg kernel, which has no tile
-  if cands[0] == 0 and len(cands) == 2:
-    cands = cands[:1]  # one tile, beside the default: nothing to choose
-  if len(cands) == 1:
-    set_launch(m, TILE, cands[0])
-    _CACHE[key] = cands[0]
-    return cands[0]
-  run = _rollout_runner(m, q, qd, acts, n_frames)
-  times = {}
-  for c in cands:
-    set_launch(m, TILE, c)
-    times[c] = _time_ms(run, reps)
-  best = min(times, key=times.get)
-  set_launch(m, TILE, best)
-  _CACHE[key] = best
-  return best
+  else:
+    _CACHE[key] = _fastest(m, TILE, cands, _rollout_runner(m, q, qd, acts, n_frames), reps)
+  return _CACHE[key]
 
 
 def tune_step(sys, q: torch.Tensor, qd: torch.Tensor, acts: torch.Tensor, n_frames: int,
               candidates: Sequence[int] = CANDIDATES, reps: int = 3) -> int:
   """Picks the envs per workgroup of the step kernels for a batch of
-  q.shape[0] envs by timing bgx_rollout over acts (T, N, act_size) from
-  copies of (q, qd); the inputs are not modified.  Returns the choice, which
-  is set on the model."""
+  q.shape[0] envs by timing a rollout over acts (T, N, act_size) from
+  (q, qd); the inputs are not modified.  A lane-per-leg kernel's workgroup is
+  one wavefront whatever the setting; on its models the rollout timed is
+  bgx_rollout_primal, the forward pass of gradients, which the setting is
+  for.  Returns the choice, which is set on the model."""
   m = pipeline.device_model(sys, q.device)
-  n = q.shape[0]
-  key = _key(m, STEP, n, n_frames)
+  key = _key(m, STEP, q.shape[0], n_frames, acts.shape[0])
   if key in _CACHE:
     set_launch(m, STEP, _CACHE[key])
-    return _CACHE[key]
-  run = _rollout_runner(m, q, qd, acts, n_frames)
-  times = {}
-  for c in candidates:
-    set_launch(m, STEP, c)
-    times[c] = _time_ms(run, reps)
-  best = min(times, key=times.get)
-  set_launch(m, STEP, best)
-  _CACHE[key] = best
-  return best
+  else:
+    _CACHE[key] = _fastest(m, STEP, candidates,
+                           _rollout_runner(m, q, qd, acts, n_frames, "bgx_rollout_primal"), reps)
+  return _CACHE[key]
 
 
 def tune_adjoint(sys, q: torch.Tensor, qd: torch.Tensor, acts: torch.Tensor, n_frames: int,
@@ -161,8 +152,7 @@ def tune_adjoint(sys, q: torch.Tensor, qd: torch.Tensor, acts: torch.Tensor, n_f
   (T, N, act_size) with one checkpoint.  Returns the choice, which is set on
   the model."""
   m = pipeline.device_model(sys, q.device)
-  n = q.shape[0]
-  key = _key(m, ADJOINT, n, n_frames)
+  key = _key(m, ADJOINT, q.shape[0], n_frames, acts.shape[0])
   if key in _CACHE:
     set_launch(m, ADJOINT, _CACHE[key])
     return _CACHE[key]
@@ -177,11 +167,5 @@ def tune_adjoint(sys, q: torch.Tensor, qd: torch.Tensor, acts: torch.Tensor, n_f
   def run():
     torch.autograd.grad((qt, qdt), (qd0, a), (gq, gqd), retain_graph=True)
 
-  times = {}
-  for c in candidates:
-    set_launch(m, ADJOINT, c)
-    times[c] = _time_ms(run, reps)
-  best = min(times, key=times.get)
-  set_launch(m, ADJOINT, best)
-  _CACHE[key] = best
-  return best
+  _CACHE[key] = _fastest(m, ADJOINT, candidates, run, reps)
+  return _CACHE[key]
