@@ -4,23 +4,21 @@
 // length up to 32 links, per-env model tables) and envs of one tree topology
 // T (shared or per-env tables).  Its envs live in packed buffers: model m's
 // envs are a contiguous range, each env's q, qd and action rows at fixed
-// strides.  The host cuts the envs into work items (64 tree envs, one per
-// lane; 16 envs of a lane per leg, bgx_star.h; or 64 / G chains of G lanes
-// each), ordered longest first, and
-// uploads the item table.  The batch rollout kernel (k_star_batch<T>, or
-// k_rollout<T, true> for other trees; k_rollout<NoTree, true> for chains
-// alone) then runs a grid of as
-// many workgroups as fit on the chip at once: each takes the next item from
-// a device counter until none is left and runs that item's envs through
-// all the rollout's substeps.  The last workgroup to leave resets the
-// counter, so the launch can be replayed (HIP graphs) without a memset.
+// strides.  The host cuts the envs into work items (16 tree envs of a lane per
+// leg, bgx_star.h; or 64 / G chains of G lanes each), ordered longest first,
+// and uploads the item table.  The batch kernel (k_star_batch<T>, or
+// k_rollout<NoTree> for chains alone) then runs a grid of as many workgroups
+// as fit on the chip at once: each takes the next item from a device counter
+// until none is left and runs that item's envs through all the rollout's
+// substeps.  The last workgroup to leave resets the counter, so the launch can
+// be replayed (HIP graphs) without a memset.
 //
-// Homogeneous launches run k_star<T> or k_rollout<T, false>
-// (k_rollout<NoTree, true> for chains), forming one item per workgroup from
-// blockIdx.  Both reach an env's substeps through the same function
-// (star_item, chain_item) or the one call site (tree_item), so an env's arithmetic is the same compiled code whether it runs alone, in
-// a batch of its kind, or in a mixed batch: results are bitwise equal at the
-// models' default launch settings (the GPU tests compare them).
+// Homogeneous launches run k_star<T> (k_rollout<NoTree> for chains), forming
+// one item per workgroup from blockIdx.  Both reach an env's substeps through
+// the same function (star_item, chain_item), so an env's arithmetic is the
+// same compiled code whether it runs alone, in a batch of its kind, or in a
+// mixed batch: results are bitwise equal at the models' default launch
+// settings (the GPU tests compare them).
 #pragma once
 
 #include <hip/hip_runtime.h>

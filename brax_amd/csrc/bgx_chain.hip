@@ -1,6 +1,6 @@
 // Kernels and launch tables of the hinge-chain topologies (bgx_chain.h: G
 // lanes per env).  One object file for every chain length: their rollouts
-// run the chain kernel k_rollout<NoTree, true> (the link count a kernel argument),
+// run the chain kernel k_rollout<NoTree> (the link count a kernel argument),
 // which also runs heterogeneous batches of chains alone; their frames a
 // kernel per lane count.  bgx.hip reaches each chain topology's table
 // through bgx_ops_<struct>().
@@ -58,7 +58,7 @@ hipError_t chain_init(const Launch& a, hipStream_t s) {
   return hipGetLastError();
 }
 
-// a homogeneous chain batch: the chain kernel (k_rollout<NoTree, true>), one item
+// a homogeneous chain batch: the chain kernel k_rollout<NoTree>, one item
 // of per envs per workgroup
 template <int L>
 hipError_t chain_rollout(const Launch& a, hipStream_t s) {
@@ -68,7 +68,7 @@ hipError_t chain_rollout(const Launch& a, hipStream_t s) {
   const int per = chain_envs_per_wg<G>(a.epw);
   Launch h = a;
   h.items = nullptr, h.chain_L = L;
-  hipLaunchKernelGGL((k_rollout<NoTree, true>), dim3((unsigned)((a.n + per - 1) / per)),
+  hipLaunchKernelGGL(k_rollout<NoTree>, dim3((unsigned)((a.n + per - 1) / per)),
                      dim3((unsigned)(per * G)), 0, s, h);
   hipError_t e = hipGetLastError();
   if (e != hipSuccess) return e;

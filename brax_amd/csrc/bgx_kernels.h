@@ -218,18 +218,11 @@ constexpr bool is_chain_kernel() {
   return std::is_same<T, NoTree>::value;
 }
 
-// LDS of the rollout kernel: the tree step's, or a chain wavefront's, or
-// the larger of the two where the kernel runs both
-template <class T, bool CHAINS>
+// LDS of the rollout kernel: the tree step's, or a chain wavefront's
+template <class T>
 constexpr int rollout_lds_floats() {
-  if constexpr (is_chain_kernel<T>()) {
-    return CHAIN_LDS_FLOATS;
-  } else if constexpr (CHAINS) {
-    return lds_floats<T>() * WAVE > CHAIN_LDS_FLOATS ? lds_floats<T>() * WAVE
-                                                      : CHAIN_LDS_FLOATS;
-  } else {
-    return lds_floats<T>() * WAVE;
-  }
+  if constexpr (is_chain_kernel<T>()) return CHAIN_LDS_FLOATS;
+  else return lds_floats<T>() * WAVE;
 }
 
 // the item of a homogeneous launch's workgroup: its envs (blockIdx.x) of
@@ -261,16 +254,14 @@ BGX_D BatchItem home_item(const Launch& a) {
   return b;
 }
 
-// The rollout kernel.  Homogeneous launch (items null): workgroup
-// (blockIdx.x, blockIdx.y) runs its own item once.  Batch launch: a
-// persistent grid; workgroups take items from the counter until the table
-// is exhausted.  T: a tree topology, or NoTree (chains only).  CHAINS: the
-// kernel also runs chain items (the batch kernel of a tree topology); its
-// tree path is the same single call site as the homogeneous kernel's, so
-// both compile it to the same arithmetic.
-template <class T, bool CHAINS>
+// The rollout kernel of a tree topology at one thread per env, or of chains (T
+// = NoTree).  Homogeneous launch (items null): workgroup (blockIdx.x,
+// blockIdx.y) runs its own item once.  Batch launch (chains alone; with trees,
+// k_star_batch): a persistent grid; workgroups take items from the counter
+// until the table is exhausted.
+template <class T>
 __global__ __launch_bounds__(WAVE) void k_rollout(Launch a) {
-  __shared__ float smem[rollout_lds_floats<T, CHAINS>()];
+  __shared__ float smem[rollout_lds_floats<T>()];
   const bool batch = a.items != nullptr;
   for (int round = 0;; ++round) {
     BatchItem b;
@@ -282,15 +273,9 @@ __global__ __launch_bounds__(WAVE) void k_rollout(Launch a) {
       if (round > 0) break;
       b = home_item<T>(a);
     }
-    if constexpr (CHAINS) {
-      if (b.kind == BATCH_CHAIN) {
-        run_chain_item(a, b, smem);
-        __syncthreads();  // the next item reuses the LDS
-        continue;
-      }
-    }
-    if constexpr (!is_chain_kernel<T>()) tree_item<T>(a, b, smem);
-    __syncthreads();
+    if constexpr (is_chain_kernel<T>()) run_chain_item(a, b, smem);
+    else tree_item<T>(a, b, smem);
+    __syncthreads();  // the next item reuses the LDS
   }
   if (batch) batch_done(a);
 }
@@ -447,13 +432,6 @@ __global__ __launch_bounds__(WAVE) void k_adj_b(AdjLaunch a) {
   }
 }
 
-// whether the topology's batch items are a lane per leg (bgx_star.h)
-template <class T>
-constexpr bool star_tree() {
-  if constexpr (is_chain_kernel<T>()) return false;
-  else return star_ok<T>();
-}
-
 // Stage B, a lane per leg: blocks of STAR_ENVS envs, coordinate-major, then
 // one thread per env for the qd coordinates (as in k_adj_b, whose time per
 // substep it had been: 77 -> 24 us for 1,024 quadrupeds off the ground, 92 ->
@@ -491,14 +469,22 @@ __global__ __launch_bounds__(WAVE) void k_star_b(AdjLaunch a) {
   if (env < a.n && b == 0) a.adj[(long long)env * ND + dir] = g;
 }
 
-// a batch launch of the rollout kernel: a persistent grid of `grid`
-// one-wavefront workgroups (a.items set)
+// the batch kernel of chains (NoTree), or of one tree topology with chains
+template <class T>
+constexpr auto batch_kernel() {
+  if constexpr (is_chain_kernel<T>()) {
+    return &k_rollout<T>;
+  } else {
+    static_assert(star_ok<T>(), "batches take trees that run a lane per leg (bgx_star.h)");
+    return &k_star_batch<T>;
+  }
+}
+
+// a batch launch: a persistent grid of `grid` one-wavefront workgroups
+// (a.items set)
 template <class T>
 hipError_t launch_batch(const Launch& a, int grid, hipStream_t s) {
-  if constexpr (star_tree<T>())
-    hipLaunchKernelGGL(k_star_batch<T>, dim3((unsigned)grid), dim3(WAVE), 0, s, a);
-  else
-    hipLaunchKernelGGL((k_rollout<T, true>), dim3((unsigned)grid), dim3(WAVE), 0, s, a);
+  hipLaunchKernelGGL(batch_kernel<T>(), dim3((unsigned)grid), dim3(WAVE), 0, s, a);
   return hipGetLastError();
 }
 
@@ -506,12 +492,8 @@ hipError_t launch_batch(const Launch& a, int grid, hipStream_t s) {
 template <class T>
 int batch_blocks_per_cu() {
   int nb = 0;
-  hipError_t e;
-  if constexpr (star_tree<T>())
-    e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&nb, k_star_batch<T>, WAVE, 0);
-  else
-    e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&nb, k_rollout<T, true>, WAVE, 0);
-  if (e != hipSuccess) return 1;
+  if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&nb, batch_kernel<T>(), WAVE, 0) != hipSuccess)
+    return 1;
   return nb > 0 ? nb : 1;
 }
 
@@ -566,7 +548,7 @@ struct Ops {
     const dim3 g = env_grid(a.n, b);
     Launch h = a;
     h.items = nullptr;
-    hipLaunchKernelGGL((k_rollout<TT, false>), dim3(g.x, a.n_seg > 1 ? (unsigned)a.n_seg : 1u),
+    hipLaunchKernelGGL(k_rollout<TT>, dim3(g.x, a.n_seg > 1 ? (unsigned)a.n_seg : 1u),
                        dim3(b), 0, s, h);
     return hipGetLastError();
   }
