@@ -118,6 +118,24 @@ def measured_traffic(kernel, name, n, steps, rel=None):
   return None
 
 
+# the committed profiles of the kernels as they are, by workload and lanes per
+# env (the quadruped's one-thread kernel and the first humanoid kernel have
+# profiles of earlier forms)
+PROFILED = {("quadruped", 4): "k_star", ("humanoid", 32): "k_mtree_rows",
+            ("humanoid", 1): "k_rollout", ("hetero", None): "k_star_batch"}
+
+
+def roofline_traffic(name, lanes, n, steps):
+  """The roofline's traffic entries: the bytes of the committed profile of
+  this launch and where they stand, or None for both."""
+  kernel = PROFILED.get((name, lanes))
+  bytes_ = measured_traffic(kernel, name, n, steps) if kernel else None
+  return {"traffic": bytes_,
+          "traffic_source": None if bytes_ is None else
+          f"{profile_path(kernel, name, n)} (rocprofv3 --pmc FETCH_SIZE, WRITE_SIZE of this "
+          "command)"}
+
+
 def host_cpu():
   """Threads the CPU baselines use (the host share this process may run on:
   OMP_NUM_THREADS when set, else the affinity mask) and a description of the
@@ -189,8 +207,6 @@ def forward_bench(args, name):
   if args.lanes:
     autotune.set_launch(m, autotune.LANES, args.lanes)
   lanes = autotune.get_launch(m, autotune.LANES)
-  # the profile's kernel: k_mtree with its mass-matrix rows in registers
-  kernel = {1: "k_rollout", 4: "k_star"}.get(lanes, "k_mtree_rows")
   if lanes > 1:
     # a multi-lane kernel's workgroup is one wavefront of 64 / lanes envs,
     # and it keeps one contact row per candidate lane (no LDS tile)
@@ -299,9 +315,7 @@ def forward_bench(args, name):
       "roofline": {"bound": "valu", "achieved": achieved,
                    "peak": FP32_PEAK_TFLOPS, "unit": "TFLOP/s",
                    "frac": achieved / FP32_PEAK_TFLOPS,
-                   "traffic": measured_traffic(kernel, name, n, K),
-                   "traffic_source": f"{profile_path(kernel, name, n)} (rocprofv3 --pmc "
-                                     "FETCH_SIZE, WRITE_SIZE of this command)",
+                   **roofline_traffic(name, lanes, n, K),
                    "flop_per_substep": fl, "mean_active_rows": r_a,
                    "mean_active_rows_source": r_a_src,
                    "kernel_ms": kernel_ms,
@@ -626,9 +640,7 @@ def hetero_bench(args):
                  "parallelism": "none (1 GPU)"},
       "roofline": {"bound": "valu", "achieved": achieved, "peak": FP32_PEAK_TFLOPS,
                    "unit": "TFLOP/s", "frac": achieved / FP32_PEAK_TFLOPS,
-                   "traffic": measured_traffic("k_star_batch", "hetero", n, K),
-                   "traffic_source": f"profiles/k_star_batch_hetero_{n}.md (rocprofv3 --pmc FETCH_SIZE, "
-                                     "WRITE_SIZE of this command)",
+                   **roofline_traffic("hetero", None, n, K),
                    "kernel_ms": kernel_ms,
                    "note": "op-count model: quadrupeds at R_a active rows, chains without rows",
                    "mean_active_rows": r_a, "mean_active_rows_source": r_a_src},
