@@ -434,8 +434,8 @@ __global__ __launch_bounds__(WAVE) void k_adj_b(AdjLaunch a) {
 
 // Stage B, a lane per leg: blocks of STAR_ENVS envs, coordinate-major, then
 // one thread per env for the qd coordinates (as in k_adj_b, whose time per
-// substep it had been: 77 -> 24 us for 1,024 quadrupeds off the ground, 92 ->
-// 47 for 2,048, 104 -> 83 for 4,096).
+// substep it had been: 78 -> 24 us for 1,024 quadrupeds off the ground, 92 ->
+// 44 for 2,048, 101 -> 81 for 4,096).
 template <class T>
 __global__ __launch_bounds__(WAVE) void k_star_b(AdjLaunch a) {
   constexpr int NQ = T::NQ, NV = T::NV, NU = T::NU, ND = NQ + NV;

@@ -11,11 +11,11 @@
 // solver's dot products) are sums over the quad, two DPP additions each with
 // no LDS and no wait.  16 envs share a wavefront.
 //
-// What bounds it: the chain of one wavefront (478 registers and 36 KB of LDS
-// for the quadruped: one wavefront per SIMD).  Before and after, one thread
-// per env and this kernel: 27 -> 7.6 us a substep off the ground for 8,192
-// quadrupeds, 72 -> 28 us for one quadruped on the floor, 140 -> 26 us for
-// 4,096 ants, 146 -> 143 us for 65,536 quadrupeds.
+// What bounds it: the chain of one wavefront (378 registers and 36 KB of LDS
+// for the quadruped: one wavefront per SIMD).  One thread per env against this
+// kernel: 27 -> 6.3 us a substep off the ground for 8,192 quadrupeds, 72 -> 21
+// us for one quadruped on the floor, 140 -> 26 us for 4,096 ants, 146 -> 109 us
+// for 65,536 quadrupeds with their frames.
 //
 // The constrained products need no tree pass: with M = L^T L the rows
 // L^-T J^T of a lane's contacts and limits are formed once per substep (they
